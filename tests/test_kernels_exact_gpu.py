@@ -342,6 +342,41 @@ def test_attention_at_the_benchmark_shapes(B, T, NH):
     G.check_no_error(L)
 
 
+@pytest.mark.parametrize("hs", [64, 80, 96, 128])
+@pytest.mark.parametrize("B,T,NH", [(1, 1, 1), (2, 31, 2), (1, 65, 3), (1, 127, 1), (1, 129, 2), (2, 192, 2), (1, 1000, 3),
+                                    (16, 500, 16), (8, 1024, 16), (1, 4200, 1)])
+def test_attention_of_any_length_and_head_size(hs, B, T, NH):
+    """Lengths around the tiles of 64 keys and 128 queries for every head size of the matrix-core kernels, launches of one and
+    of two query tiles per workgroup (the last three have workgroups to spare), and a length whose statistics do not fit LDS.
+    The fp32 formulation, relative Frobenius error. out of the wide heads: P is carried to 2^-17, so what is left is the
+    rounding of the result, at most 2^-9 = 1.95e-3 of each element. Their gradients add what rounding O to bf16 does to
+    D = rowsum(dO O), of the same size: 4e-3. A head size of 64 rounds P and dS to bf16 too: 1e-2 as at the benchmark shapes."""
+    import torch
+    L = G.lib("bf16")
+    Cc = NH * hs
+    gen = torch.Generator(device="cuda"); gen.manual_seed(B * T + hs)
+    qkv = torch.randn((B, T, 3 * Cc), generator=gen, device="cuda").to(torch.bfloat16)
+    dout = torch.randn((B, T, Cc), generator=gen, device="cuda").to(torch.bfloat16)
+    out = torch.zeros((B, T, Cc), dtype=torch.bfloat16, device="cuda")
+    stats = torch.zeros((B, NH, T), dtype=torch.float32, device="cuda")
+    dqkv = torch.full((B, T, 3 * Cc), 3.0, dtype=torch.bfloat16, device="cuda")
+    print("attention", hs, B, T, NH, flush=True)
+    L.llmk_attention_forward(G.ptr(out), G.ptr(stats), G.ptr(qkv), B, T, NH, Cc, None)
+    L.llmk_attention_backward(G.ptr(dqkv), G.ptr(dout), G.ptr(qkv), G.ptr(out), G.ptr(stats), B, T, NH, Cc, None)
+    G.sync()
+    r_out, r_lse, r_d = torch_attention(qkv, dout, NH)
+    wide = hs != 64
+    assert rel_fro(out, r_out) < (2.2e-3 if wide else 1e-2)
+    # a row's log-sum-exp: fp32 sums of P to 2^-17 (wide), of P rounded to 2^-9 (64)
+    assert (stats - r_lse).abs().max().item() < (1e-4 if wide else 2e-2)
+    d, rd = dqkv.float().view(B, T, 3, NH, hs), r_d.view(B, T, 3, NH, hs)
+    joint = rd.pow(2).sum((1, 2, 4)).sqrt()                      # per (batch, head): no single head is off
+    for i, name in enumerate(("dQ", "dK", "dV")):
+        e = ((d[:, :, i] - rd[:, :, i]).pow(2).sum((1, 3)).sqrt() / joint).max().item()
+        assert e < (4e-3 if wide else 1e-2), (name, e)
+    G.check_no_error(L)
+
+
 @pytest.mark.parametrize("pattern", ["random", "rising", "falling"])
 @pytest.mark.parametrize("T", [1024, 320])
 def test_attention_with_large_scores(T, pattern):
