@@ -19,6 +19,7 @@
 // fp32 build: straightforward one-wave-per-row kernels (lanes = head dimensions), used only for
 // parity runs against the CPU reference at small sizes.
 #include "common.hpp"
+#include "decode.hpp"
 #include <type_traits>
 #include <utility>
 #include "../../include/llmk.h"
@@ -342,14 +343,14 @@ constexpr float FA_MAX_SLACK = 8.0f;
 // for the tile in flight.
 // RAGGED: T is not a multiple of 128, so the last tiles of a head are cut (see fa_tile_request); the same arithmetic in
 // the same order, so a row's bits do not depend on which of the two it went through.
-// Workgroups take one query tile or two (nq tiles per head, grid.x of them or half as many): see fa_tiles_paired.
+// Workgroups take one query tile or two (nq tiles per head): see fa_tiles_paired.
 // Measured against the one-wave-per-row kernels that the heads of 80, 96 and 128 used to take, whose every score is a 64-lane
 // reduction on the vector ALU (2 x 2048 x 16 heads of 128, us): forward 15348 -> 92 (375 TFLOP/s of the causal half), dQ
 // 15684 -> 114, dK/dV 17177 -> 189; 3 x 1000 x 16 heads of 96: 4705 -> 43, 4845 -> 52, 5708 -> 65. What bounds them now: two
 // waves per SIMD (registers), a third of the matrix work being the low parts of P and dS.
 template <int HD, bool RAGGED>
 __global__ void __launch_bounds__(256, HD == 64 ? 4 : 2)
-fa_forward_dma_kernel(floatX* __restrict__ out, float* __restrict__ stats, const floatX* __restrict__ qkv, int T, int NH, int nq) {
+fa_forward_dma_kernel(floatX* __restrict__ out, float* __restrict__ stats, const floatX* __restrict__ qkv, int T, int NH, int nq, bool paired) {
     constexpr int NWAVES = 4;
     constexpr int KS = FaTile<HD>::KS, NB = FaTile<HD>::NB;
     __shared__ __attribute__((aligned(1024))) char sK[2][FaTile<HD>::BYTES];
@@ -362,7 +363,7 @@ fa_forward_dma_kernel(floatX* __restrict__ out, float* __restrict__ stats, const
     // second tile's first keys are already on their way when the first tile is stored. Launches too small for that take
     // one, the longest first.
     const int qt_first = nq - 1 - tile_x, qt_second = tile_x;
-    const int nphase = qt_first == qt_second || (int)gridDim.x == nq ? 1 : 2;
+    const int nphase = qt_first == qt_second || !paired ? 1 : 2;
     const int b = bh / NH, h = bh % NH;
     const int C = NH * HD;
     const size_t C3 = 3 * (size_t)C;
@@ -527,7 +528,7 @@ fa_forward_dma_kernel(floatX* __restrict__ out, float* __restrict__ stats, const
 template <int HD, bool RAGGED, bool LDS_STATS>
 __global__ void __launch_bounds__(256, HD == 64 ? 1 : 2)
 fa_backward_dkdv_dma_kernel(floatX* __restrict__ dqkv, const floatX* __restrict__ dout, const floatX* __restrict__ qkv,
-                        const float* __restrict__ stats, const float* __restrict__ Dsum, int T, int NH, int nk) {
+                        const float* __restrict__ stats, const float* __restrict__ Dsum, int T, int NH, int nk, bool paired) {
     constexpr int KS = FaTile<HD>::KS, NB = FaTile<HD>::NB;
     constexpr int SLOT = HD == 64 ? SW_TILE : 2 * SW_TILE;       // the power of two that holds a tile
     static_assert(FaTile<HD>::SLOT <= SLOT, "a tile fits its slot");
@@ -545,7 +546,7 @@ fa_backward_dkdv_dma_kernel(floatX* __restrict__ dqkv, const floatX* __restrict_
     // coincide): equal work for every workgroup of the launch, and the second tile's first queries are on their way
     // when the first tile is stored. Launches too small for that take one.
     const int kt_first = tile_x, kt_second = nk - 1 - tile_x;
-    const int nphase = kt_first == kt_second || (int)gridDim.x == nk ? 1 : 2;
+    const int nphase = kt_first == kt_second || !paired ? 1 : 2;
     const int b = bh / NH, h = bh % NH;
     const int C = NH * HD;
     const size_t C3 = 3 * (size_t)C;
@@ -759,7 +760,7 @@ template <int HD, bool RAGGED>
 __global__ void __launch_bounds__(256, HD == 64 ? 4 : 2)
 fa_backward_dq_dma_kernel(floatX* __restrict__ dqkv, const floatX* __restrict__ dout, const floatX* __restrict__ qkv,
                           const floatX* __restrict__ o, const float* __restrict__ stats, float* __restrict__ Dsum, int T, int NH,
-                          int nq) {
+                          int nq, bool paired) {
     constexpr int KS = FaTile<HD>::KS, NB = FaTile<HD>::NB;
     __shared__ __attribute__((aligned(1024))) char sK[2][FaTile<HD>::SLOT];
     __shared__ __attribute__((aligned(1024))) char sV[2][FaTile<HD>::BYTES];
@@ -768,7 +769,7 @@ fa_backward_dq_dma_kernel(floatX* __restrict__ dqkv, const floatX* __restrict__ 
     fa_block_coords(tile_x, bh);
     // two query tiles per workgroup, nq - 1 - x and then x, as in fa_forward_dma_kernel: equal work for every workgroup (or one)
     const int qt_first = nq - 1 - tile_x, qt_second = tile_x;
-    const int nphase = qt_first == qt_second || (int)gridDim.x == nq ? 1 : 2;
+    const int nphase = qt_first == qt_second || !paired ? 1 : 2;
     const int b = bh / NH, h = bh % NH;
     const int C = NH * HD;
     const size_t C3 = 3 * (size_t)C;
@@ -912,11 +913,11 @@ fa_backward_dq_dma_kernel(floatX* __restrict__ dqkv, const floatX* __restrict__ 
 template <int EPL>
 __global__ void __launch_bounds__(256)
 att_forward_rows_kernel(floatX* __restrict__ out, float* __restrict__ stats, const floatX* __restrict__ qkv, int B, int T,
-                        int NH, int hs) {
-    const int lane = threadIdx.x & 63;
+                        int NH, int hs, int t0) {
+    const int lane = threadIdx.x & 63, nt = T - t0;                       // positions t0 .. T - 1 of every head
     const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);       // (b, h, t)
-    if (row >= (size_t)B * NH * T) return;
-    const int t = (int)(row % T), h = (int)((row / T) % NH), b = (int)(row / ((size_t)T * NH));
+    if (row >= (size_t)B * NH * nt) return;
+    const int t = t0 + (int)(row % nt), h = (int)((row / nt) % NH), b = (int)(row / ((size_t)nt * NH));
     const int C = NH * hs;
     const size_t C3 = 3 * (size_t)C;
     const floatX* base = qkv + (size_t)b * T * C3 + h * hs;
@@ -1055,10 +1056,10 @@ att_backward_dkdv_rows_kernel(floatX* __restrict__ dqkv, const floatX* __restric
         }
 }
 
-void launch_forward_rows(floatX* out, float* stats, const floatX* qkv, int B, int T, int NH, int hs, hipStream_t st) {
-    const unsigned blocks = (unsigned)CEIL_DIV((size_t)B * NH * T, (size_t)4);
-    if (hs <= 64) att_forward_rows_kernel<1><<<blocks, 256, 0, st>>>(out, stats, qkv, B, T, NH, hs);
-    else att_forward_rows_kernel<2><<<blocks, 256, 0, st>>>(out, stats, qkv, B, T, NH, hs);
+void launch_forward_rows(floatX* out, float* stats, const floatX* qkv, int B, int T, int NH, int hs, int t0, hipStream_t st) {
+    const unsigned blocks = (unsigned)CEIL_DIV((size_t)B * NH * (T - t0), (size_t)4);
+    if (hs <= 64) att_forward_rows_kernel<1><<<blocks, 256, 0, st>>>(out, stats, qkv, B, T, NH, hs, t0);
+    else att_forward_rows_kernel<2><<<blocks, 256, 0, st>>>(out, stats, qkv, B, T, NH, hs, t0);
 }
 void launch_backward_rows(floatX* dqkv, const floatX* dout, const floatX* qkv, const floatX* o, const float* stats, int B,
                           int T, int NH, int hs, hipStream_t st) {
@@ -1112,19 +1113,25 @@ bool fa_tiles_paired(int ntiles, int nbh) {
 
 template <int HD, bool RAGGED>
 void launch_fa_forward(floatX* out, float* stats, const floatX* qkv, int B, int T, int NH, hipStream_t st) {
-    const int nq = CEIL_DIV(T, 128), gx = fa_tiles_paired(nq, B * NH) ? (nq + 1) / 2 : nq;
-    fa_forward_dma_kernel<HD, RAGGED><<<dim3(gx, B * NH), 256, 0, st>>>(out, stats, qkv, T, NH, nq);
+    const int nq = CEIL_DIV(T, 128);
+    const bool paired = fa_tiles_paired(nq, B * NH);
+    const int gx = paired ? (nq + 1) / 2 : nq;
+    fa_forward_dma_kernel<HD, RAGGED><<<dim3(gx, B * NH), 256, 0, st>>>(out, stats, qkv, T, NH, nq, paired);
 }
 template <int HD, bool RAGGED>
 void launch_fa_dq(floatX* dqkv, const floatX* dout, const floatX* qkv, const floatX* o, const float* stats, float* Dsum, int B, int T,
                   int NH, hipStream_t st) {
-    const int nq = CEIL_DIV(T, 128), gx = fa_tiles_paired(nq, B * NH) ? (nq + 1) / 2 : nq;
-    fa_backward_dq_dma_kernel<HD, RAGGED><<<dim3(gx, B * NH), 256, 0, st>>>(dqkv, dout, qkv, o, stats, Dsum, T, NH, nq);
+    const int nq = CEIL_DIV(T, 128);
+    const bool paired = fa_tiles_paired(nq, B * NH);
+    const int gx = paired ? (nq + 1) / 2 : nq;
+    fa_backward_dq_dma_kernel<HD, RAGGED><<<dim3(gx, B * NH), 256, 0, st>>>(dqkv, dout, qkv, o, stats, Dsum, T, NH, nq, paired);
 }
 template <int HD, bool RAGGED>
 void launch_fa_dkdv(floatX* dqkv, const floatX* dout, const floatX* qkv, const float* stats, const float* Dsum, int B, int T, int NH,
                     hipStream_t st) {
-    const int nk = CEIL_DIV(T, 128), gx = fa_tiles_paired(nk, B * NH) ? (nk + 1) / 2 : nk;
+    const int nk = CEIL_DIV(T, 128);
+    const bool paired = fa_tiles_paired(nk, B * NH);
+    const int gx = paired ? (nk + 1) / 2 : nk;
     const dim3 grid(gx, B * NH);
     if (T <= 4096) {                              // 2 T floats of statistics (32 KiB at most) beside the 32 or 64 KiB of tiles
         const size_t dyn = 2 * (size_t)CEIL_DIV(T, 64) * 64 * sizeof(float);
@@ -1134,9 +1141,9 @@ void launch_fa_dkdv(floatX* dqkv, const floatX* dout, const floatX* qkv, const f
             HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 4096 * (int)sizeof(float)));
             attr_set = true;
         }
-        kern<<<grid, 256, dyn, st>>>(dqkv, dout, qkv, stats, Dsum, T, NH, nk);
+        kern<<<grid, 256, dyn, st>>>(dqkv, dout, qkv, stats, Dsum, T, NH, nk, paired);
     } else {
-        fa_backward_dkdv_dma_kernel<HD, RAGGED, false><<<grid, 256, 0, st>>>(dqkv, dout, qkv, stats, Dsum, T, NH, nk);
+        fa_backward_dkdv_dma_kernel<HD, RAGGED, false><<<grid, 256, 0, st>>>(dqkv, dout, qkv, stats, Dsum, T, NH, nk, paired);
     }
 }
 // the head sizes of the GPT-2 and GPT-3 models run on the matrix cores (the direct-to-LDS loads and the stores of a lane need
@@ -1192,6 +1199,23 @@ void attention_backward_impl(void* dqkvr, const void* dout, const void* qkvr, co
 
 namespace llmk {
 void attention_static_scratch_init() { (void)static_scratch_setup(); }
+
+// One sequence, queries t0 .. T - 1 (t0 a multiple of 32, T - t0 at most 32) against keys 0 .. T - 1, with the bits that a
+// sampled token has always depended on. Heads of 64: the matrix-core kernel runs the query tile that holds the rows, one
+// workgroup per head; the rows of that tile before t0 come out again as they were. Others: one wave per row.
+void decode_attention(void* out, const void* qkv, int t0, int T, int NH, int C, hipStream_t st) {
+    if (failed()) return;
+    const int hs = C / NH;
+#if !defined(LLMK_FP32)
+    if (hs == 64) {
+        fa_forward_dma_kernel<64, true><<<dim3(1, NH), 256, 0, st>>>((floatX*)out, nullptr, (const floatX*)qkv, T, NH, CEIL_DIV(T, 128), false);
+        LAUNCH_CHECK();
+        return;
+    }
+#endif
+    launch_forward_rows((floatX*)out, nullptr, (const floatX*)qkv, 1, T, NH, hs, t0, st);
+    LAUNCH_CHECK();
+}
 }  // namespace llmk
 
 extern "C" {
@@ -1220,7 +1244,7 @@ void llmk_attention_forward(void* out, float* stats, const void* inp, int B, int
         return;
     }
 #endif
-    launch_forward_rows((floatX*)out, stats, (const floatX*)inp, B, T, NH, hs, st);
+    launch_forward_rows((floatX*)out, stats, (const floatX*)inp, B, T, NH, hs, 0, st);
     LAUNCH_CHECK();
 }
 

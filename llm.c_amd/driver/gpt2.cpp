@@ -24,6 +24,7 @@
 #include "../../include/llmk.h"
 #include "../../include/llmk_gpt2.h"
 #include "../../include/llmk_data.h"
+#include "../csrc/decode.hpp"
 #include "rand.hpp"
 
 #define hipCheck(expr)                                                                            \
@@ -93,6 +94,7 @@ struct LLMK_GPT2 {
     int gelu_fusion = 0, recompute = 1;
     int* workload_indices = nullptr;
     int* bucket_info = nullptr;
+    char* decode_host = nullptr;               // pinned: the 32 tokens and the logits row of a generation step
     hipStream_t stream = nullptr;
 };
 
@@ -522,23 +524,78 @@ float gpt2_validate(LLMK_GPT2* m, const int* inputs, const int* targets, size_t 
     return mean_loss / (float)(B * T);
 }
 
+namespace {
+constexpr int DECODE_ROWS = 32;                // rows of one generation step: the row block of the matrix kernels
+
+// The forward pass of positions r0 .. r0 + n - 1 of one sequence (r0 a multiple of DECODE_ROWS, n at most that) whose earlier
+// positions have been through here: their K and V lie in the qkvr tensor, layer by layer, seq_len rows each. Everything else
+// is needed for these rows only and goes through the first rows of the activation tensors. A row's result depends on its own
+// inputs and the K and V before it, and every kernel adds up in the order of the full forward pass: the same bits. Leaves the
+// logits of the rows at output + r0 rows. tokens: device-visible, the n tokens.
+void decode_block(LLMK_GPT2* m, const int* tokens, int r0, int n) {
+    const size_t Vp = m->config.padded_vocab_size, L = m->config.num_layers, C = m->config.channels, X = m->X, T = m->seq_len;
+    const int NH = m->config.num_heads;
+    hipStream_t st = m->stream;
+    const ParameterTensors p = m->params;
+    const ActivationTensors a = m->acts;
+    const xptr ln = a.lnf, atty = off(a.atty, (size_t)r0 * C, X), scratch = a.output;
+    llmk_encoder_forward(a.encoded, tokens, p.wte, off(p.wpe, (size_t)r0 * C, X), 1, n, (int)C, st);
+    llmk_layernorm_forward(ln, nullptr, nullptr, a.encoded, p.ln1w, p.ln1b, 1, n, (int)C, st);
+    xptr residual = a.encoded;
+    for (size_t l = 0; l < L; l++) {
+        const xptr qkv = off(a.qkvr, l * T * 3 * C, X);
+        llmk::decode_matmul(off(qkv, (size_t)r0 * 3 * C, X), ln, off(p.qkvw, l * 3 * C * C, X), off(p.qkvb, l * 3 * C, X), nullptr, nullptr,
+                            n, (int)C, (int)(3 * C), st);
+        llmk::decode_attention(a.atty, qkv, r0, r0 + n, NH, (int)C, st);
+        const xptr n_w = l + 1 != L ? off(p.ln1w, (l + 1) * C, X) : p.lnfw, n_b = l + 1 != L ? off(p.ln1b, (l + 1) * C, X) : p.lnfb;
+        const xptr ln2w = off(p.ln2w, l * C, X), ln2b = off(p.ln2b, l * C, X);
+        const xptr attprojw = off(p.attprojw, l * C * C, X), attprojb = off(p.attprojb, l * C, X);
+        const xptr fcw = off(p.fcw, l * 4 * C * C, X), fcb = off(p.fcb, l * 4 * C, X);
+        const xptr fcprojw = off(p.fcprojw, l * C * 4 * C, X), fcprojb = off(p.fcprojb, l * C, X);
+        if (X == 2) {                              // as in forward_impl: the adds are the projections' epilogues
+            llmk::decode_matmul(a.residual2, atty, attprojw, attprojb, nullptr, residual, n, (int)C, (int)C, st);
+            llmk_layernorm_forward(ln, nullptr, nullptr, a.residual2, ln2w, ln2b, 1, n, (int)C, st);
+            llmk::decode_matmul(a.fch_gelu, ln, fcw, fcb, a.fch, nullptr, n, (int)C, (int)(4 * C), st);
+            llmk::decode_matmul(a.residual3, a.fch_gelu, fcprojw, fcprojb, nullptr, a.residual2, n, (int)(4 * C), (int)C, st);
+            llmk_layernorm_forward(ln, nullptr, nullptr, a.residual3, n_w, n_b, 1, n, (int)C, st);
+        } else {
+            llmk::decode_matmul(scratch, atty, attprojw, attprojb, nullptr, nullptr, n, (int)C, (int)C, st);
+            llmk_fused_residual_forward5(a.residual2, ln, nullptr, nullptr, residual, scratch, ln2w, ln2b, n, (int)C, st);
+            llmk::decode_matmul(a.fch_gelu, ln, fcw, fcb, a.fch, nullptr, n, (int)C, (int)(4 * C), st);
+            llmk::decode_matmul(scratch, a.fch_gelu, fcprojw, fcprojb, nullptr, nullptr, n, (int)(4 * C), (int)C, st);
+            llmk_fused_residual_forward5(a.residual3, ln, nullptr, nullptr, a.residual2, scratch, n_w, n_b, n, (int)C, st);
+        }
+        residual = a.residual3;
+    }
+    llmk::decode_matmul(off(a.output, (size_t)r0 * Vp, X), ln, p.wte, nullptr, nullptr, nullptr, n, (int)C, (int)Vp, st);
+}
+}  // namespace
+
 // The generation loop of the reference's trainer (train_gpt2.cu:1751-1796), without the printing: every position of
 // gen_tokens starts as eot_token, then positions 1..genT-1 are drawn one at a time from the model's distribution after
-// the tokens before them. Each draw runs the forward pass on one sequence whose length is rounded up to a multiple of
-// min(seq_len, 256) (no KV cache, as there), moves the logits of the last real position to the host and samples there
-// with llmc/sampler.h's generator, whose state the caller owns (the reference starts it at 1337 for every generation).
+// the tokens before them. The reference runs the whole sequence, rounded up to a multiple of 256, for every draw; here a draw
+// runs the block of 32 rows that its position lies in, on the K and V of the rows before (decode_block). The logits of the last
+// real position move to the host and are sampled there with llmc/sampler.h's generator, whose state the caller owns (the
+// reference starts it at 1337 for every generation).
 void gpt2_generate(LLMK_GPT2* m, int* gen_tokens, int genT, int eot_token, unsigned long long* sample_rng_state) {
     const int B = m->batch_size, T = m->seq_len, V = m->config.vocab_size;
     const size_t Vp = m->config.padded_vocab_size;
+    if (m->params_memory == nullptr) { printf("Error: model was not initialized properly.\n"); exit(EXIT_FAILURE); }
     if (genT > T) { printf("gpt2_generate: genT=%d exceeds the sequence length %d\n", genT, T); exit(EXIT_FAILURE); }
     for (int i = 0; i < B * T; i++) gen_tokens[i] = eot_token;
-    std::vector<char> raw((size_t)V * m->X);
+    if (genT > 1) token_check(&eot_token, 1, V);
+    const size_t row_bytes = (size_t)V * m->X;
+    if (!m->decode_host) hipCheck(hipHostMalloc((void**)&m->decode_host, DECODE_ROWS * sizeof(int) + row_bytes));
+    int* tokens = (int*)m->decode_host;
+    char* raw = m->decode_host + DECODE_ROWS * sizeof(int);
     std::vector<float> cpu_logits(V);
-    const int chunk = T < 256 ? T : 256;
     for (int t = 1; t < genT; t++) {
-        gpt2_forward(m, gen_tokens, 1, (size_t)((t + chunk - 1) / chunk) * chunk);
-        hipCheck(hipMemcpy(raw.data(), off(m->acts.output, (size_t)(t - 1) * Vp, m->X), (size_t)V * m->X, hipMemcpyDeviceToHost));
-        from_storage(cpu_logits.data(), raw.data(), V, m->X);
+        const int r0 = (t - 1) / DECODE_ROWS * DECODE_ROWS, n = std::min(DECODE_ROWS, T - r0);
+        memcpy(tokens, gen_tokens + r0, n * sizeof(int));      // the stream is idle here: the step before has been waited for
+        decode_block(m, tokens, r0, n);
+        hipCheck(hipMemcpyAsync(raw, off(m->acts.output, (size_t)(t - 1) * Vp, m->X), row_bytes, hipMemcpyDeviceToHost, m->stream));
+        hipCheck(hipStreamSynchronize(m->stream));
+        from_storage(cpu_logits.data(), raw, V, m->X);
         const float coin = llmk::random_f32(sample_rng_state);
         gen_tokens[t] = llmk::sample_softmax(cpu_logits.data(), V, coin);
     }
@@ -783,6 +840,7 @@ void gpt2_free(LLMK_GPT2* m) {
     if (m->cpu_losses) (void)hipHostFree(m->cpu_losses);
     if (m->workload_indices) (void)hipHostFree(m->workload_indices);
     if (m->bucket_info) (void)hipHostFree(m->bucket_info);
+    if (m->decode_host) (void)hipHostFree(m->decode_host);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
 }

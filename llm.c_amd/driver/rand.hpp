@@ -102,13 +102,15 @@ inline float random_f32(unsigned long long* state) { return (random_u32(state) >
 
 // Index drawn from softmax(logits) with the uniform number `coin` (reference: llmc/sampler.h:22-40): the
 // normaliser is summed in double, the running distribution in float, and the coin is scaled instead of the terms.
-inline int sample_softmax(const float* logits, int n, float coin) {
+// The logits are overwritten with their exponentials (the reference evaluates each of them twice).
+inline int sample_softmax(float* logits, int n, float coin) {
+    for (int i = 0; i < n; i++) logits[i] = expf(logits[i]);
     double norm = 0;
-    for (int i = 0; i < n; i++) norm += expf(logits[i]);
+    for (int i = 0; i < n; i++) norm += logits[i];
     coin *= norm;
     float cdf = 0.0f;
     for (int i = 0; i < n; i++) {
-        cdf += expf(logits[i]);
+        cdf += logits[i];
         if (coin < cdf) return i;
     }
     return n - 1;

@@ -484,6 +484,42 @@ def test_bf16_generation_samples_from_its_own_logits():
     m.free()
 
 
+@pytest.mark.parametrize("precision,cfg,T,genT", [
+    ("bf16", (160, 300, 320, 2, 2, 128), 150, 150),      # heads of 64; the last block of 32 rows is cut off by the sequence's end
+    ("bf16", (128, 300, 320, 2, 2, 192), 128, 70),       # heads of 96: one wave per row
+    ("bf16", (64, 300, 320, 2, 3, 120), 64, 40),         # channels that the generation kernels do not take
+    ("fp32", (160, 300, 320, 2, 2, 128), 150, 70),
+])
+def test_generation_by_blocks_is_the_full_forward_pass(precision, cfg, T, genT):
+    """Every draw of gpt2_generate runs the block of 32 rows that its position lies in, on the K and V kept from the rows
+    before. Each token has to be the sampler's answer for that position's logits of a full forward pass over the finished
+    sequence. Against the full pass the bf16 logits may round differently (other kernels, other order of sums), which
+    moves a token only when a coin falls within that rounding of a boundary of the distribution: 3 of them at most, and none
+    in fp32."""
+    cfg = ol.Config(*cfg)
+    eot = cfg.vocab_size - 1
+    params = np.ascontiguousarray(ol.init_params(cfg, 11) * np.float32(8), np.float32)
+    m = Model(precision, cfg, 1, T, params=params)
+    tokens = np.zeros(T, np.int32)
+    state = C.c_ulonglong(1337)
+    m.L.gpt2_generate(m.h, tokens.ctypes.data_as(C.c_void_p), genT, eot, C.byref(state))
+    assert tokens[0] == eot and (tokens[genT:] == eot).all() and len(set(tokens[1:genT].tolist())) > 10
+    m.L.gpt2_forward(m.h, tokens.ctypes.data_as(C.c_void_p), 1, T)
+    lg = m.logits(cfg.padded_vocab_size).reshape(T, cfg.padded_vocab_size)
+    st = C.c_uint64(1337)
+    off = 0
+    for t in range(1, genT):
+        coin = ol.cref().cref_random_f32(C.byref(st))
+        off += ol.cref().cref_sample_softmax(np.ascontiguousarray(lg[t - 1, :cfg.vocab_size]), cfg.vocab_size, coin) != tokens[t]
+    assert off <= (3 if precision == "bf16" else 0), off
+    # a second generation on the same model starts over
+    again = np.zeros(T, np.int32)
+    state = C.c_ulonglong(1337)
+    m.L.gpt2_generate(m.h, again.ctypes.data_as(C.c_void_p), genT, eot, C.byref(state))
+    np.testing.assert_array_equal(again, tokens)
+    m.free()
+
+
 def full_size_steps(cfg, B, T, recompute, gelu_fusion, steps=3, want_wte=True, lr=6e-4, whole_step=False):
     """A few AdamW steps at a shape the oracle cannot run, with what must hold at any size checked on the way: the
     initial loss (the final LayerNorm gives unit-variance channels and wte is N(0, 0.02), so the logits of a position
