@@ -18,7 +18,7 @@
  *   - no entry point here allocates device memory per call. Two launchers take scratch from ONE
  *     library-owned workspace (the role of the reference's cublaslt_workspace,
  *     llmc/cublas_common.h:28-31): llmk_matmul_backward (fp32 partial products of the split
- *     weight gradient) and llmk_attention_backward (one float per query and head). The
+ *     weight gradient and, for few rows, of dinp) and llmk_attention_backward (one float per query and head). The
  *     workspace grows to the largest request seen (a free, an allocation and a device
  *     synchronisation at that call) and is then reused; a caller that must not allocate inside
  *     a step sizes it beforehand with llmk_workspace_reserve() from the

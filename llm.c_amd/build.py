@@ -21,7 +21,7 @@ LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(HERE, "build")
 
 KERNEL_SOURCES = ["runtime.hip", "layernorm.hip", "gelu.hip", "encoder.hip", "classifier.hip", "optimizer.hip",
-                  "gemm.hip", "gemm_tn.hip", "decode.hip", "attention.hip"]
+                  "gemm.hip", "gemm_tn.hip", "gemm_ring.hip", "decode.hip", "attention.hip"]
 # options of single files: the weight-gradient GEMM kernels take the compiler's "max-ilp" instruction scheduling (measured
 # per kernel family, each variant loaded beside the product in one process: these kernels -1.2 to -2.7 %, every other GEMM
 # kernel +2 to +8 %, attention forward -1.5 %, dQ 0, dK/dV +9 %)
@@ -30,6 +30,7 @@ KERNEL_SOURCES = ["runtime.hip", "layernorm.hip", "gelu.hip", "encoder.hip", "cl
 # dK/dV -1.5 %, forward and dQ unchanged; top-down only: every GEMM kernel +10 to +19 %).
 FILE_FLAGS = {"gemm_tn.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
               "gemm.hip": ["-mllvm", "-misched-prera-direction=bottomup"],
+              "gemm_ring.hip": ["-mllvm", "-misched-prera-direction=bottomup"],
               "attention.hip": ["-mllvm", "-misched-prera-direction=bottomup"]}
 DRIVER_SOURCES = ["gpt2.cpp", "data.cpp"]
 

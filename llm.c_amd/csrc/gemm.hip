@@ -22,11 +22,14 @@
 //   * dweight has few output tiles (27 for 2304x768) but K = 65536: the contraction is split
 //     over workgroups, partials go to the library workspace in fp32 and are added in split
 //     order by a second kernel (deterministic; no atomics), which also does the += into dW.
+//   * launches of few tiles take the ring kernels (gemm_ring.hip), by estimated time (plan_gemm)
 // fp32 build: same structure with v_mfma_f32_32x32x2_f32 (true fp32 multiply-add), the mode
 // used for 1e-5 parity against the CPU reference.
 #include "common.hpp"
 #include "gelu.hpp"
 #include "gemm_pipelined.hpp"
+#include "gemm_ring.hpp"
+#include <limits>
 #include <vector>
 #include <algorithm>
 #include "../../include/llmk.h"
@@ -263,11 +266,12 @@ constexpr int BIG_TILE = 256, SMALL_TILE = 128, K_STEP = 64;
 
 // Persistent direct-to-LDS kernel (gemm_pipelined.hpp). Preconditions: K and the per-split K multiples of 32,
 // leading dimensions and N multiples of 8, 16-byte aligned operands, 8-byte aligned bias.
-bool pipelined_ok(const GemmArgs& g) {
+bool operands_ok(const GemmArgs& g) {
     auto al = [](const void* p, uintptr_t a) { return ((uintptr_t)p % a) == 0; };
-    return g.K % KGRAN == 0 && g.k_per_split % KGRAN == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.ldc % 8 == 0 &&
-           g.N % 8 == 0 && al(g.A, 16) && al(g.B, 16) && al(g.C, 16) && (!g.bias || al(g.bias, 8)) && (!g.aux || al(g.aux, 16));
+    return g.lda % 8 == 0 && g.ldb % 8 == 0 && g.ldc % 8 == 0 && g.N % 8 == 0 && al(g.A, 16) && al(g.B, 16) && al(g.C, 16) &&
+           (!g.bias || al(g.bias, 8)) && (!g.aux || al(g.aux, 16));
 }
+bool pipelined_ok(const GemmArgs& g) { return g.K % KGRAN == 0 && g.k_per_split % KGRAN == 0 && operands_ok(g); }
 // The pipelined kernel's += epilogue spills registers (it holds the old values of a whole tile); with it available,
 // a single "split" written as fp32 partials and folded in by the reduce pass is 30 % faster than accumulating in place.
 bool tn_partial_always(const GemmArgs& g) { return pipelined_ok(g); }
@@ -301,6 +305,18 @@ template <bool A_T, bool B_T, int EPI>
 void launch_best(const GemmArgs& g, int splits, bool big, hipStream_t st) {
     if (pipelined_ok(g)) launch_pipelined<A_T, B_T, EPI>(g, splits, big, st);
     else launch_gemm<A_T, B_T, EPI>(g, splits, big, st);
+}
+constexpr int DINP_MAX_SPLITS = 32, DWEIGHT_MAX_SPLITS = 16;
+// forward: K in one piece, so that a row's sums are taken in one order at every batch size (and no scratch is needed)
+template <int EPI>
+bool launch_forward(const GemmArgs& g, hipStream_t st) {
+    constexpr bool SMALL_TILES = EPI == EPI_BIAS || EPI == EPI_STORE || EPI == EPI_BIAS_GELU;
+    if (!pipelined_ok(g)) return false;
+    const GemmPlan plan = plan_gemm(0, g.M, g.N, g.K, 1, SMALL_TILES, 0, llmk::device_info().num_cu);
+    if (plan.kernel >= 0) launch_ring(plan, g, false, false, EPI, nullptr, st);
+    else if constexpr (SMALL_TILES) launch_pipelined<false, false, EPI>(g, 1, plan.kernel == PERSISTENT_BIG, st);
+    else launch_pipelined_cfg<256, 256, 2, 4, false, false, EPI>(g, 1, st);
+    return true;
 }
 
 #else
@@ -431,13 +447,14 @@ void launch_best(const GemmArgs& g, int splits, bool big, hipStream_t st) { laun
 bool tn_partial_always(const GemmArgs&) { return false; }
 #endif
 
+enum { SKR_STORE = 0, SKR_ACCUM = 1, SKR_DGELU = 2, SKR_DGELU_D = 3 };    // (the last two: times gelu'(aux), times aux)
 // C[m][n] (+)= sum over splits of partial[s][m][n], in split order. Workgroups past the ones that cover C add up the
 // row sums of EPI_PARTIAL_ROWSUM: rowvec[m] += sum over parts of rowsum[p][m], 32 rows per workgroup, 8 groups of lanes
 // each adding every 8th part, then the 8 sub-sums in group order (a fixed tree, like bias_grad_reduce_kernel).
 constexpr int SKR_ROWS = 32, SKR_GROUPS = 8;
-template <bool ACCUM>
+template <int MODE>
 __global__ void __launch_bounds__(256)
-splitk_reduce_kernel(floatX* __restrict__ C, const float* __restrict__ partial, size_t mn, int splits,
+splitk_reduce_kernel(floatX* __restrict__ C, const floatX* __restrict__ aux, const float* __restrict__ partial, size_t mn, int splits,
                      floatX* __restrict__ rowvec, const float* __restrict__ rowsum, int rows, int parts, unsigned main_blocks) {
     if (blockIdx.x >= main_blocks) {                      // workgroup-uniform
         __shared__ float sub[SKR_GROUPS][SKR_ROWS];
@@ -466,8 +483,12 @@ splitk_reduce_kernel(floatX* __restrict__ C, const float* __restrict__ partial, 
     }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        float base = ACCUM ? to_f32(C[i + e]) : 0.f;
-        C[i + e] = from_f32<floatX>(base + s[e]);
+        if (MODE == SKR_ACCUM) C[i + e] = from_f32<floatX>(to_f32(C[i + e]) + s[e]);
+        else {
+            const floatX d = from_f32<floatX>(s[e]);              // rounded before the product, as a separate pass would see it
+            if (MODE == SKR_STORE) C[i + e] = d;
+            else C[i + e] = from_f32<floatX>((MODE == SKR_DGELU_D ? to_f32(aux[i + e]) : gelu_grad_f(to_f32(aux[i + e]))) * to_f32(d));
+        }
     }
 }
 
@@ -527,6 +548,21 @@ int tn_equal_splits(int M, size_t tiles, int num_cu, double* cost_out) {
     splits = min(splits, max(1, ksteps / 8));                     // at least 8 K steps per split
     return CEIL_DIV(ksteps, CEIL_DIV(ksteps, splits));
 }
+
+#if !defined(LLMK_FP32)
+// The weight gradient dW[OC][C] over M rows: the persistent kernel and its pass over partial products against the ring
+// kernels, which also take a number of rows that is not a multiple of 64
+GemmPlan dweight_plan(int M, int C, int OC, int num_cu) {
+    const size_t big_tiles = (size_t)CEIL_DIV(OC, BIG_TILE) * CEIL_DIV(C, BIG_TILE);
+    const bool big = big_tiles >= 8;
+    double us = std::numeric_limits<double>::infinity();
+    if (M % K_STEP == 0) {
+        const size_t tiles = big ? big_tiles : (size_t)CEIL_DIV(OC, SMALL_TILE) * CEIL_DIV(C, SMALL_TILE);
+        us = persistent_tn_us(OC, C, M, tn_equal_splits(M, tiles, num_cu, nullptr), big, num_cu);
+    }
+    return plan_gemm(2, OC, C, M, DWEIGHT_MAX_SPLITS, false, us, num_cu);
+}
+#endif
 
 // what the last weight-gradient GEMM did with K: 0 = not cut, 1 = equal splits, 2 = one long + short pieces
 int g_last_split_kind = 0, g_last_split_pieces = 0;
@@ -696,18 +732,15 @@ void llmk_matmul_forward(void* out, const void* inp, const void* weight, const v
     g.A = (const floatX*)inp; g.B = (const floatX*)weight; g.M = M; g.N = OC; g.K = C;
     g.lda = C; g.ldb = C; g.ldc = OC; g.bias = (const floatX*)bias; g.k_per_split = CEIL_DIV(C, K_STEP) * K_STEP;
     const int num_cu = llmk::device_info().num_cu;
-    const bool big = (size_t)CEIL_DIV(M, BIG_TILE) * CEIL_DIV(OC, BIG_TILE) >= (size_t)num_cu;
+    const bool big = (size_t)CEIL_DIV(M, BIG_TILE) * CEIL_DIV(OC, BIG_TILE) >= (size_t)num_cu;    // (generic kernels)
     const bool gelu_in_gemm = pre_gelu && gelu_fusion >= 1;            // then the kernel writes two (M, OC) tensors
     llmk::ProfScope prof(gelu_in_gemm ? "gemm_nt_gelu" : "gemm_nt", 2.0 * M * (double)OC * C,
                          ((double)M * C + (double)OC * C + (gelu_in_gemm ? 2.0 : 1.0) * M * OC) * sizeof(floatX), st);
     if (pre_gelu && gelu_fusion >= 3) {
-        // pre_gelu receives gelu'(pre-activation): in the direct-to-LDS kernel's epilogue, else by a pass of its own
+        // pre_gelu receives gelu'(pre-activation): in the epilogue of the direct-to-LDS kernels, else by a pass of its own
         g.C = (floatX*)out; g.aux = (floatX*)pre_gelu;
 #if !defined(LLMK_FP32)
-        if (big && pipelined_ok(g)) {
-            launch_pipelined_cfg<256, 256, 2, 4, false, false, EPI_BIAS_GELU_D>(g, 1, st);
-            return;
-        }
+        if (launch_forward<EPI_BIAS_GELU_D>(g, st)) return;
 #endif
         g.C = (floatX*)pre_gelu; g.aux = nullptr;
         launch_best<false, false, EPI_BIAS>(g, 1, big, st);
@@ -715,16 +748,24 @@ void llmk_matmul_forward(void* out, const void* inp, const void* weight, const v
         llmk_gelu_forward_keep_grad(out, pre_gelu, M * OC, stream);
     } else if (pre_gelu && gelu_fusion >= 1) {
         g.C = (floatX*)out; g.aux = (floatX*)pre_gelu;
+#if !defined(LLMK_FP32)
+        if (launch_forward<EPI_BIAS_GELU>(g, st)) return;
+#endif
         launch_best<false, false, EPI_BIAS_GELU>(g, 1, big, st);
-    } else if (pre_gelu) {
-        g.C = (floatX*)pre_gelu;
-        launch_best<false, false, EPI_BIAS>(g, 1, big, st);
-        if (prof.on) { llmk::prof_end(st); prof.on = false; }
-        llmk_gelu_forward(out, pre_gelu, M * OC, stream);
     } else {
-        g.C = (floatX*)out;
-        if (bias) launch_best<false, false, EPI_BIAS>(g, 1, big, st);
-        else launch_best<false, false, EPI_STORE>(g, 1, big, st);     // the LM head: no bias to fetch, no window to keep for it
+        g.C = (floatX*)(pre_gelu ? pre_gelu : out);
+#if !defined(LLMK_FP32)
+        const bool done = bias ? launch_forward<EPI_BIAS>(g, st) : launch_forward<EPI_STORE>(g, st);   // the LM head: no bias to fetch, no window to keep for it
+#else
+        const bool done = false;
+#endif
+        if (done) {
+        } else if (bias) launch_best<false, false, EPI_BIAS>(g, 1, big, st);
+        else launch_best<false, false, EPI_STORE>(g, 1, big, st);
+        if (pre_gelu) {
+            if (prof.on) { llmk::prof_end(st); prof.on = false; }
+            llmk_gelu_forward(out, pre_gelu, M * OC, stream);
+        }
     }
 }
 
@@ -765,13 +806,17 @@ size_t llmk_matmul_backward_workspace_bytes(int B, int T, int C, int OC) {
     const size_t tiles_big = (size_t)CEIL_DIV(OC, BIG_TILE) * CEIL_DIV(C, BIG_TILE);
     const size_t tiles_small = (size_t)CEIL_DIV(OC, SMALL_TILE) * CEIL_DIV(C, SMALL_TILE);
     int pieces = tn_equal_splits(M, tiles_big >= 8 ? tiles_big : tiles_small, num_cu, nullptr);
+    size_t dinp = 0;
 #if !defined(LLMK_FP32)
     if (tiles_big >= 8 && M % K_STEP == 0) {
         const SkPlan plan = sk_build(CEIL_DIV(OC, BIG_TILE), CEIL_DIV(C, BIG_TILE), M / K_STEP, num_cu & ~7, 800.0 / (double)M);
         if (plan.valid) pieces = max(pieces, plan.slots);
     }
+    pieces = max(pieces, dweight_plan(M, C, OC, num_cu).splits);
+    const int dinp_pieces = plan_gemm(1, M, C, OC, DINP_MAX_SPLITS, true, 0, num_cu).splits;
+    if (dinp_pieces > 1) dinp = (size_t)M * C * dinp_pieces * sizeof(float);
 #endif
-    return ((size_t)OC * C + (size_t)OC * 4) * pieces * sizeof(float);     // partial products + the bias gradient's row sums
+    return max(dinp, ((size_t)OC * C + (size_t)OC * 4) * pieces * sizeof(float));     // partial products + the bias gradient's row sums
 }
 
 // out = bf16(bf16(inp . weight^T + bias) + residual): the projection and the residual stream's add in one launch, with
@@ -790,10 +835,9 @@ void llmk_matmul_forward_residual(void* out, const void* inp, const void* weight
     g.A = (const floatX*)inp; g.B = (const floatX*)weight; g.M = M; g.N = OC; g.K = C;
     g.lda = C; g.ldb = C; g.ldc = OC; g.bias = (const floatX*)bias; g.k_per_split = CEIL_DIV(C, K_STEP) * K_STEP;
     g.C = (floatX*)out; g.aux = (floatX*)residual;
-    const bool big = (size_t)CEIL_DIV(M, BIG_TILE) * CEIL_DIV(OC, BIG_TILE) >= (size_t)llmk::device_info().num_cu;
-    if (big && out != residual && aligned16(residual) && aligned16(out) && pipelined_ok(g)) {
+    if (out != residual && aligned16(residual) && aligned16(out) && pipelined_ok(g)) {
         llmk::ProfScope prof("gemm_nt_res", 2.0 * M * (double)OC * C, ((double)M * C + (double)OC * C + 2.0 * M * OC) * sizeof(floatX), st);
-        launch_pipelined_cfg<256, 256, 2, 4, false, false, EPI_BIAS_RES>(g, 1, st);
+        launch_forward<EPI_BIAS_RES>(g, st);
         return;
     }
 #endif
@@ -820,11 +864,14 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
     // pass over dout. Same preconditions as that kernel; otherwise the streaming reduction in (1).
     bool dbias_in_gemm = false;
 #if !defined(LLMK_FP32)
-    if (dbias) {
+    GemmPlan dw_plan;                    // of the ring kernels, or left at the persistent one's
+    {
         GemmArgs t{};
         t.A = (const floatX*)dout; t.B = (const floatX*)inp; t.C = (floatX*)dweight;
         t.M = OC; t.N = C; t.K = M; t.lda = OC; t.ldb = C; t.ldc = C; t.k_per_split = KGRAN;
-        dbias_in_gemm = pipelined_ok(t) && M % K_STEP == 0;
+        if (operands_ok(t) && g_sk_mode < 0) dw_plan = dweight_plan(M, C, OC, num_cu);
+        dbias_in_gemm = dbias && (dw_plan.kernel >= 0 || pipelined_ok(t));
+        LLMK_REQUIRE(!dbias || pipelined_ok(t) || dbias_buffer != nullptr, "matmul_backward: dbias_buffer is required when dbias is given");
     }
 #endif
 
@@ -850,25 +897,42 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
 #if defined(LLMK_FP32)
         const bool fused = pre_gelu && gelu_fusion >= 2 && !stored_grad;
 #else
-        // bf16: gelu' goes into the epilogue of the direct-to-LDS kernel (big tiles only); the bias gradient of the layer
+        // bf16: gelu' goes into the epilogue of the direct-to-LDS kernels; the bias gradient of the layer
         // below then comes out of its weight-gradient GEMM, and no elementwise pass over (B,T,4C) is left
-        const bool fused = pre_gelu && gelu_fusion >= 2 && big && aligned16(pre_gelu) && pipelined_ok(g);
+        const bool fused = pre_gelu && gelu_fusion >= 2 && aligned16(pre_gelu) && pipelined_ok(g);
+        GemmPlan plan;
+        if (pipelined_ok(g)) plan = plan_gemm(1, M, C, OC, DINP_MAX_SPLITS, !fused, 0, num_cu);
 #endif
         {
             // with GELU backward in the epilogue the kernel also reads the (M, C) pre-activations
             llmk::ProfScope prof(fused ? "gemm_nn_dgelu" : "gemm_nn", 2.0 * M * (double)OC * C,
                                  ((double)M * OC + (double)OC * C + (fused ? 2.0 : 1.0) * M * C) * sizeof(floatX), st);
-            if (fused) {
-                g.aux = (floatX*)pre_gelu;
+            if (fused) g.aux = (floatX*)pre_gelu;
 #if defined(LLMK_FP32)
-                launch_best<false, true, EPI_DGELU>(g, 1, big, st);
+            if (fused) launch_best<false, true, EPI_DGELU>(g, 1, big, st);
+            else launch_best<false, true, EPI_STORE>(g, 1, big, st);
 #else
+            if (plan.kernel >= 0 && plan.splits > 1) {
+                const size_t mn = (size_t)M * C;
+                g.partial = (float*)llmk::workspace(mn * plan.splits * sizeof(float));
+                launch_ring(plan, g, false, true, EPI_PARTIAL, nullptr, st);
+                auto reduce = [&](auto kern) {
+                    const unsigned blocks = (unsigned)CEIL_DIV(mn / 4, (size_t)256);
+                    kern<<<blocks, 256, 0, st>>>(g.C, g.aux, g.partial, mn, plan.splits, nullptr, nullptr, 0, 0, blocks);
+                };
+                if (!fused) reduce(splitk_reduce_kernel<SKR_STORE>);
+                else if (stored_grad) reduce(splitk_reduce_kernel<SKR_DGELU_D>);
+                else reduce(splitk_reduce_kernel<SKR_DGELU>);
+                LAUNCH_CHECK();
+            } else if (plan.kernel >= 0) {
+                launch_ring(plan, g, false, true, !fused ? EPI_STORE : stored_grad ? EPI_DGELU_D : EPI_DGELU, nullptr, st);
+            } else if (fused) {
                 if (stored_grad) launch_pipelined_cfg<256, 256, 2, 4, false, true, EPI_DGELU_D>(g, 1, st);
                 else launch_pipelined_cfg<256, 256, 2, 4, false, true, EPI_DGELU>(g, 1, st);
-#endif
             } else {
-                launch_best<false, true, EPI_STORE>(g, 1, big, st);
+                launch_best<false, true, EPI_STORE>(g, 1, pipelined_ok(g) ? plan.kernel == PERSISTENT_BIG : big, st);
             }
+#endif
         }
         if (pre_gelu && !fused) {
             if (stored_grad) llmk_gelu_backward_from_grad(dinp, pre_gelu, M * C, stream);
@@ -889,6 +953,26 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
         const int splits = tn_equal_splits(M, tiles, num_cu, &best_uniform);
         g.k_per_split = CEIL_DIV(CEIL_DIV(M, K_STEP), splits) * K_STEP;
         const double tn_bytes = ((double)M * OC + (double)M * C + 2.0 * OC * C) * sizeof(floatX);
+#if !defined(LLMK_FP32)
+        if (dw_plan.kernel >= 0) {
+            const int pieces = dw_plan.splits;
+            const size_t mn = (size_t)OC * C;
+            g_last_split_kind = pieces > 1 ? 1 : 0; g_last_split_pieces = pieces;
+            if (pieces > 1) g.partial = (float*)llmk::workspace((mn + (size_t)OC) * pieces * sizeof(float));
+            if (pieces > 1 && dbias) g.rowsum = g.partial + mn * pieces;                 // [pieces][OC]
+            {
+                llmk::ProfScope prof(pieces > 1 ? "gemm_tn_splitk" : "gemm_tn", 2.0 * M * (double)OC * C, tn_bytes, st);
+                launch_ring(dw_plan, g, true, true, pieces == 1 ? EPI_ACCUM : dbias ? EPI_PARTIAL_ROWSUM : EPI_PARTIAL, (floatX*)dbias, st);
+            }
+            if (pieces == 1) return;
+            llmk::ProfScope prof("splitk_reduce", 0, (double)mn * pieces * sizeof(float) + 2.0 * mn * sizeof(floatX), st);
+            const unsigned main_blocks = (unsigned)CEIL_DIV(mn / 4, (size_t)256), bias_blocks = dbias ? (unsigned)CEIL_DIV(OC, SKR_ROWS) : 0u;
+            splitk_reduce_kernel<SKR_ACCUM><<<main_blocks + bias_blocks, 256, 0, st>>>((floatX*)dweight, nullptr, g.partial, mn, pieces,
+                                                                                     (floatX*)dbias, g.rowsum, OC, pieces, main_blocks);
+            LAUNCH_CHECK();
+            return;
+        }
+#endif
         if (splits == 1 && !tn_partial_always(g)) {
             LLMK_REQUIRE(!dbias_in_gemm, "matmul_backward: bias gradient was left to a kernel that is not being run");
             llmk::ProfScope prof("gemm_tn", 2.0 * M * (double)OC * C, tn_bytes, st);
@@ -915,7 +999,7 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
             llmk::ProfScope prof("splitk_reduce", 0, (double)mn * slots * sizeof(float) + 2.0 * mn * sizeof(floatX), st);
             const unsigned main_blocks = (unsigned)CEIL_DIV(mn / 4, (size_t)256);
             const unsigned bias_blocks = dbias_in_gemm ? (unsigned)CEIL_DIV(OC, SKR_ROWS) : 0u;
-            splitk_reduce_kernel<true><<<main_blocks + bias_blocks, 256, 0, st>>>((floatX*)dweight, g.partial, mn, slots,
+            splitk_reduce_kernel<SKR_ACCUM><<<main_blocks + bias_blocks, 256, 0, st>>>((floatX*)dweight, nullptr, g.partial, mn, slots,
                                                                                (floatX*)dbias, g.rowsum, OC, slots * parts, main_blocks);
             LAUNCH_CHECK();
 #endif
@@ -939,7 +1023,7 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
             llmk::ProfScope prof("splitk_reduce", 0, (double)mn * splits * sizeof(float) + 2.0 * mn * sizeof(floatX), st);
             const unsigned main_blocks = (unsigned)CEIL_DIV(mn / 4, (size_t)256);
             const unsigned bias_blocks = dbias_in_gemm ? (unsigned)CEIL_DIV(OC, SKR_ROWS) : 0u;
-            splitk_reduce_kernel<true><<<main_blocks + bias_blocks, 256, 0, st>>>((floatX*)dweight, g.partial, mn, splits,
+            splitk_reduce_kernel<SKR_ACCUM><<<main_blocks + bias_blocks, 256, 0, st>>>((floatX*)dweight, nullptr, g.partial, mn, splits,
                                                                                (floatX*)dbias, g.rowsum, OC, splits * parts, main_blocks);
             LAUNCH_CHECK();
         }

@@ -222,6 +222,59 @@ def _backward_projection_case(L, C, OC):
     G.check_no_error(L)
 
 
+# Launches of few output tiles: one row, ragged rows at every tile height, a partly filled and several filled rounds of
+# workgroups, column counts that end inside a tile, contractions of one stage, of a cut last stage (rows as K) and long enough to
+# be cut into pieces
+FEW_TILES = [(1, 64, 72), (63, 128, 64), (200, 768, 2304), (333, 384, 1536), (65, 384, 50304), (1000, 1600, 832), (1000, 6400, 1600),
+             (2331, 384, 1152), (2331, 1536, 384), (3000, 1536, 4608), (4096, 2048, 2048), (4160, 768, 768), (777, 3072, 1024)]
+
+
+@pytest.mark.parametrize("M,C,OC", FEW_TILES)
+def test_projections_of_few_tiles_are_the_integer_products(M, C, OC):
+    """Forward with each epilogue, dinp with and without GELU backward, dweight and dbias, at sizes that leave part of the chip
+    idle: every product exact, every fused epilogue the same bits as the pass of its own that it stands for."""
+    import torch
+    L = G.lib("bf16")
+    x, w, b = ints((M, C), 21, -2, 2), ints((OC, C), 22), ints((OC,), 23, -8, 8)
+    lin = exact_nt(x, w) + b.float()
+    out = torch.full((M, OC), 7.0, dtype=torch.bfloat16, device="cuda")
+    L.llmk_matmul_forward(G.ptr(out), G.ptr(x), G.ptr(w), G.ptr(b), 1, M, C, OC, None, None, 1)
+    G.sync()
+    assert_same_bits(out, lin, "x.w^T + b")
+    res = (torch.randn((M, OC), device="cuda") * 3.0).to(torch.bfloat16)
+    L.llmk_matmul_forward_residual(G.ptr(out), G.ptr(x), G.ptr(w), G.ptr(b), G.ptr(res), 1, M, C, OC, None)
+    G.sync()
+    assert_same_bits(out, lin.to(torch.bfloat16).float() + res.float(), "x.w^T + b + residual")
+    ws = ints((OC, C), 22, scale=1.0 / 32)
+    pre_want = (exact_nt(x, ws) + b.float()).to(torch.bfloat16)
+    act_want, grad_want = torch.empty_like(out), torch.ones_like(out)
+    L.llmk_gelu_forward(G.ptr(act_want), G.ptr(pre_want), M * OC, None)
+    L.llmk_gelu_backward_inplace(G.ptr(grad_want), G.ptr(pre_want), M * OC, None)
+    for fusion, kept in ((0, pre_want), (1, pre_want), (2, pre_want), (3, grad_want)):
+        pre = torch.zeros_like(out)
+        L.llmk_matmul_forward(G.ptr(out), G.ptr(x), G.ptr(ws), G.ptr(b), 1, M, C, OC, None, G.ptr(pre), fusion)
+        G.sync()
+        assert torch.equal(pre, kept) and torch.equal(out, act_want), fusion
+    g = ints((M, OC), 24, -2, 2)
+    dw0, db0 = ints((OC, C), 25, -50, 50), ints((OC,), 26, -50, 50)
+    scratch = torch.empty(max(1, L.llmk_matmul_backward_bias_scratch_floats(OC)), dtype=torch.float32, device="cuda")
+    dx_want = exact_nt(g, w.t().contiguous())
+    dw_want, db_want = dw0.float() + exact_tn(g, x), db0.float() + g.float().sum(0)
+    kept = ints((M, C), 27, -24, 24, scale=1.0 / 8)
+    for fusion in (None, 0, 2, 3):
+        dx, dw, db = torch.full((M, C), 7.0, dtype=torch.bfloat16, device="cuda"), dw0.clone(), db0.clone()
+        L.llmk_matmul_backward(G.ptr(dx), G.ptr(dw), G.ptr(db) if fusion != 2 else None, G.ptr(g), G.ptr(x), G.ptr(w), G.ptr(scratch),
+                               1, M, C, OC, None, None if fusion is None else G.ptr(kept), 1 if fusion is None else fusion)
+        want = dx_want.to(torch.bfloat16)
+        if fusion == 3: want = (want.float() * kept.float()).to(torch.bfloat16)
+        elif fusion is not None: L.llmk_gelu_backward_inplace(G.ptr(want), G.ptr(kept), M * C, None)
+        G.sync()
+        assert torch.equal(dx, want), ("dinp", fusion)
+        assert_same_bits(dw, dw_want, "dweight")
+        assert_same_bits(db, db_want if fusion != 2 else db0.float(), "dbias")
+    G.check_no_error(L)
+
+
 @pytest.mark.parametrize("C,OC", [(3072, 768), (4096, 1024), (6400, 1600)])
 def test_backward_projection_with_gelu_epilogue(C, OC):
     """The fcproj layer's dinp with GELU backward in the GEMM's epilogue (gelu_fusion 2): the product of the once-rounded
