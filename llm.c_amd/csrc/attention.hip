@@ -16,8 +16,8 @@
 // Two kernels instead of one with atomics: every output element has exactly one owner, so the
 // result is deterministic, as the reference requests from cuDNN (cudnn_att.cpp:187-189).
 //
-// fp32 build: straightforward one-wave-per-row kernels (lanes = head dimensions), used only for
-// parity runs against the CPU reference at small sizes.
+// fp32 build: the same on the fp32 matrix instruction for heads of 32, 64, 96 and 128; other head sizes of either build take
+// one-wave-per-row kernels (lanes = head dimensions).
 #include "common.hpp"
 #include "decode.hpp"
 #include <type_traits>
@@ -907,8 +907,8 @@ fa_backward_dq_dma_kernel(floatX* __restrict__ dqkv, const floatX* __restrict__ 
 
 // =============================================================================================
 // Any head size up to 128, either storage type: one wavefront per row, lane l holds head dimensions l and l + 64
-// (EPL = 2) or l alone (EPL = 1, hs <= 64). All arithmetic in fp32. The fp32 build's only path; the bf16 build takes
-// it for the head sizes its MFMA kernels do not cover (none of the descriptors', train_gpt2.cu:519-559).
+// (EPL = 2) or l alone (EPL = 1, hs <= 64). All arithmetic in fp32. For the head sizes
+// that the MFMA kernels do not cover (none of the descriptors', train_gpt2.cu:519-559).
 // =============================================================================================
 template <int EPL>
 __global__ void __launch_bounds__(256)
@@ -1056,13 +1056,307 @@ att_backward_dkdv_rows_kernel(floatX* __restrict__ dqkv, const floatX* __restric
         }
 }
 
+#if defined(LLMK_FP32)
+// =============================================================================================
+// fp32 build, heads of 32, 64, 96 and 128: the same two-kernel
+// scheme as the bf16 build on v_mfma_f32_32x32x2_f32, true fp32 multiply-adds. A wave owns 32 queries (forward, dQ) or 32 keys
+// (dK/dV), two waves share the 32-row tiles of the other side in LDS; the next tile is on its way in registers meanwhile.
+//   * The contraction over head dimensions may take them in any order as long as both operands agree: lane half h holds dims
+//     8 j + 4 h .. + 3 of its row, one 16-byte read for four matrix instructions.
+//   * A 32 x 32 accumulator gives lane l column l % 32 and rows 8 g + 4 (l / 32) + e: as the second operand of the next product, its
+//     register 4 g + e is the k pair (8 g + e, 8 g + 4 + e), so probabilities go from one product into the next without moving.
+//   * Probabilities of masked positions are zeros that are multiplied like any other, as in the bf16 kernels.
+// What bounds it: one dependent chain of matrix instructions per wave (64 cycles each) with the exponentials between; the
+// one-wave-per-row kernels it replaces spend two 64-lane reductions per score.
+// =============================================================================================
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+constexpr int F_ROWS = 64, F_THREADS = 128;                       // rows of a workgroup (32 per wave)
+
+// 32 rows x HD floats of a matrix with `ld` floats between rows, rows past the last one repeating it
+template <int HD>
+struct F32Tile {
+    static constexpr int PITCH = HD + 4;                          // 16 rows' 16-byte reads cover all banks
+    static constexpr int FLOATS = 32 * PITCH, N = 32 * HD / 4 / F_THREADS;
+    f32x4 reg[N];
+    __device__ __forceinline__ void load(const float* base, size_t ld, int r0, int rows) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int q = (int)threadIdx.x + i * F_THREADS, row = q / (HD / 4), c = q % (HD / 4);
+            reg[i] = *reinterpret_cast<const f32x4*>(base + (size_t)min(r0 + row, rows - 1) * ld + c * 4);
+        }
+    }
+    __device__ __forceinline__ void store(float* lds) const {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int q = (int)threadIdx.x + i * F_THREADS, row = q / (HD / 4), c = q % (HD / 4);
+            *reinterpret_cast<f32x4*>(lds + row * PITCH + c * 4) = reg[i];
+        }
+    }
+};
+template <int HD> using F32Row = f32x4[HD / 8];
+template <int HD>
+__device__ __forceinline__ void f32_row(F32Row<HD>& r, const float* row, int half) {
+#pragma unroll
+    for (int j = 0; j < HD / 8; j++) r[j] = *reinterpret_cast<const f32x4*>(row + 8 * j + 4 * half);
+}
+// rows of the LDS tile (accumulator rows) against this lane's row (accumulator column)
+template <int HD>
+__device__ __forceinline__ f32x16 f32_scores(const float* tile, const F32Row<HD>& mine, int lane) {
+    const float* row = tile + (lane & 31) * F32Tile<HD>::PITCH + 4 * (lane >> 5);
+    f32x16 a;
+#pragma unroll
+    for (int r = 0; r < 16; r++) a[r] = 0.f;
+#pragma unroll
+    for (int j = 0; j < HD / 8; j++) {
+        const f32x4 t = *reinterpret_cast<const f32x4*>(row + 8 * j);
+#pragma unroll
+        for (int e = 0; e < 4; e++) a = __builtin_amdgcn_mfma_f32_32x32x2f32(t[e], mine[j][e], a, 0, 0, 0);
+    }
+    return a;
+}
+// acc[d] (rows: head dims 32 d ..) += tile^T . p, contracted over the tile's 32 rows
+template <int HD>
+__device__ __forceinline__ void f32_accumulate(f32x16 (&acc)[HD / 32], const float* tile, const f32x16& p, int lane) {
+    const float* at = tile + 4 * (lane >> 5) * F32Tile<HD>::PITCH + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+        for (int d = 0; d < HD / 32; d++)
+            acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(at[(8 * (r >> 2) + (r & 3)) * F32Tile<HD>::PITCH + 32 * d], p[r], acc[d], 0, 0, 0);
+}
+// the lane's column of an accumulator over head dims to its row in memory
+template <int HD>
+__device__ __forceinline__ void f32_store(float* row, const f32x16 (&acc)[HD / 32], float denominator, int half) {
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const f32x4 o = {acc[d][4 * g] / denominator, acc[d][4 * g + 1] / denominator, acc[d][4 * g + 2] / denominator, acc[d][4 * g + 3] / denominator};
+            *reinterpret_cast<f32x4*>(row + 32 * d + 8 * g + 4 * half) = o;
+        }
+}
+
+// queries q_first + 64 x ..; blocks of the later ones, which have more keys, are dealt first
+template <int HD>
+__global__ void __launch_bounds__(F_THREADS)
+att_forward_f32_kernel(float* __restrict__ out, float* __restrict__ stats, const float* __restrict__ qkv, int T, int NH, int q_first) {
+    __shared__ __attribute__((aligned(16))) float sk[F32Tile<HD>::FLOATS], sv[F32Tile<HD>::FLOATS];
+    const int lane = threadIdx.x & 63, half = lane >> 5, wave = threadIdx.x >> 6;
+    const int b = blockIdx.y / NH, h = blockIdx.y % NH, C = NH * HD;
+    const size_t C3 = 3 * (size_t)C;
+    const float* base = qkv + (size_t)b * T * C3 + h * HD;
+    const int w0 = q_first + (int)(gridDim.x - 1 - blockIdx.x) * F_ROWS, q0 = w0 + wave * 32, q = q0 + (lane & 31);
+    const float scale = 1.0f / sqrtf((float)HD);
+    F32Row<HD> mine;
+    f32_row<HD>(mine, base + (size_t)min(q, T - 1) * C3, half);
+    f32x16 acc[HD / 32];
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[d][r] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    const int kend = min(w0 + F_ROWS, T);                         // keys of the workgroup's last query
+    F32Tile<HD> tk, tv;
+    tk.load(base + C, C3, 0, T);
+    tv.load(base + 2 * C, C3, 0, T);
+    for (int k0 = 0; k0 < kend; k0 += 32) {
+        __syncthreads();
+        tk.store(sk);
+        tv.store(sv);
+        __syncthreads();
+        if (k0 + 32 < kend) {
+            tk.load(base + C, C3, k0 + 32, T);
+            tv.load(base + 2 * C, C3, k0 + 32, T);
+        }
+        if (k0 > q0) continue;                                    // the first wave is done a block earlier
+        f32x16 s = f32_scores<HD>(sk, mine, lane);
+        float top = m;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            s[r] *= scale;
+            if (k0 == q0 && (r >> 2) * 8 + 4 * half + (r & 3) > (lane & 31)) s[r] = -INFINITY;
+            top = fmaxf(top, s[r]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const float alpha = expf(m - top);
+        float sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) { s[r] = expf(s[r] - top); sum += s[r]; }
+        l = l * alpha + (sum + __shfl_xor(sum, 32, 64));
+        m = top;
+#pragma unroll
+        for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[d][r] *= alpha;
+        f32_accumulate<HD>(acc, sv, s, lane);
+    }
+    if (q >= T) return;
+    f32_store<HD>(out + ((size_t)b * T + q) * C + h * HD, acc, l, half);
+    if (stats && half == 0) stats[((size_t)b * NH + h) * T + q] = m + logf(l);
+}
+
+template <int HD>
+__global__ void __launch_bounds__(F_THREADS)
+att_backward_dq_f32_kernel(float* __restrict__ dqkv, const float* __restrict__ dout, const float* __restrict__ qkv,
+                           const float* __restrict__ o, const float* __restrict__ stats, int T, int NH) {
+    __shared__ __attribute__((aligned(16))) float sk[F32Tile<HD>::FLOATS], sv[F32Tile<HD>::FLOATS];
+    const int lane = threadIdx.x & 63, half = lane >> 5, wave = threadIdx.x >> 6;
+    const int b = blockIdx.y / NH, h = blockIdx.y % NH, C = NH * HD;
+    const size_t C3 = 3 * (size_t)C;
+    const float* base = qkv + (size_t)b * T * C3 + h * HD;
+    const int w0 = (int)(gridDim.x - 1 - blockIdx.x) * F_ROWS, q0 = w0 + wave * 32, q = q0 + (lane & 31), qc = min(q, T - 1);
+    const float scale = 1.0f / sqrtf((float)HD);
+    const size_t orow = ((size_t)b * T + qc) * C + h * HD;
+    F32Row<HD> mine, go;
+    f32_row<HD>(mine, base + (size_t)qc * C3, half);
+    f32_row<HD>(go, dout + orow, half);
+    float dsum = 0.f;
+    {
+        F32Row<HD> fo;
+        f32_row<HD>(fo, o + orow, half);
+#pragma unroll
+        for (int j = 0; j < HD / 8; j++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) dsum += go[j][e] * fo[j][e];
+        dsum += __shfl_xor(dsum, 32, 64);
+    }
+    const float lse = stats[((size_t)b * NH + h) * T + qc];
+    f32x16 acc[HD / 32];
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[d][r] = 0.f;
+    const int kend = min(w0 + F_ROWS, T);
+    F32Tile<HD> tk, tv;
+    tk.load(base + C, C3, 0, T);
+    tv.load(base + 2 * C, C3, 0, T);
+    for (int k0 = 0; k0 < kend; k0 += 32) {
+        __syncthreads();
+        tk.store(sk);
+        tv.store(sv);
+        __syncthreads();
+        if (k0 + 32 < kend) {
+            tk.load(base + C, C3, k0 + 32, T);
+            tv.load(base + 2 * C, C3, k0 + 32, T);
+        }
+        if (k0 > q0) continue;
+        f32x16 p = f32_scores<HD>(sk, mine, lane);
+        const f32x16 dp = f32_scores<HD>(sv, go, lane);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const bool masked = k0 == q0 && (r >> 2) * 8 + 4 * half + (r & 3) > (lane & 31);
+            p[r] = masked ? 0.f : expf(p[r] * scale - lse) * (dp[r] - dsum) * scale;
+        }
+        f32_accumulate<HD>(acc, sk, p, lane);
+    }
+    if (q < T) f32_store<HD>(dqkv + ((size_t)b * T + q) * C3 + h * HD, acc, 1.0f, half);
+}
+
+template <int HD>
+__global__ void __launch_bounds__(F_THREADS)
+att_backward_dkdv_f32_kernel(float* __restrict__ dqkv, const float* __restrict__ dout, const float* __restrict__ qkv,
+                             const float* __restrict__ o, const float* __restrict__ stats, int T, int NH) {
+    __shared__ __attribute__((aligned(16))) float sq[F32Tile<HD>::FLOATS], sg[F32Tile<HD>::FLOATS], sl[32], sd[32];
+    const int lane = threadIdx.x & 63, half = lane >> 5, wave = threadIdx.x >> 6;
+    const int b = blockIdx.y / NH, h = blockIdx.y % NH, C = NH * HD;
+    const size_t C3 = 3 * (size_t)C;
+    const float* base = qkv + (size_t)b * T * C3 + h * HD;
+    const float *gbase = dout + (size_t)b * T * C + h * HD, *obase = o + (size_t)b * T * C + h * HD;
+    const float* lbase = stats + ((size_t)b * NH + h) * T;
+    const int w0 = (int)blockIdx.x * F_ROWS, k0 = w0 + wave * 32, k = k0 + (lane & 31), kc = min(k, T - 1);
+    const float scale = 1.0f / sqrtf((float)HD);
+    F32Row<HD> mk, mv;
+    f32_row<HD>(mk, base + C + (size_t)kc * C3, half);
+    f32_row<HD>(mv, base + 2 * C + (size_t)kc * C3, half);
+    f32x16 dk[HD / 32], dv[HD / 32];
+#pragma unroll
+    for (int d = 0; d < HD / 32; d++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) dk[d][r] = dv[d][r] = 0.f;
+    F32Tile<HD> tq, tg;
+    tq.load(base, C3, w0, T);
+    tg.load(gbase, C, w0, T);
+    float lse = 0.f, dsum = 0.f;
+    auto load_rows = [&](int t0) {                                // D = rowsum(dO * O): four threads to a row
+        const int row = (int)threadIdx.x >> 2, part = threadIdx.x & 3;
+        const size_t at = (size_t)min(t0 + row, T - 1) * C + part * (HD / 4);
+        float s = 0.f;
+#pragma unroll
+        for (int c = 0; c < HD / 4; c += 4) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(gbase + at + c), y = *reinterpret_cast<const f32x4*>(obase + at + c);
+#pragma unroll
+            for (int e = 0; e < 4; e++) s += x[e] * y[e];
+        }
+        s += __shfl_xor(s, 1, 64);
+        dsum = s + __shfl_xor(s, 2, 64);
+        lse = lbase[min(t0 + row, T - 1)];
+    };
+    load_rows(w0);
+    for (int t0 = w0; t0 < T; t0 += 32) {
+        __syncthreads();
+        tq.store(sq);
+        tg.store(sg);
+        if ((threadIdx.x & 3) == 0) { sl[threadIdx.x >> 2] = lse; sd[threadIdx.x >> 2] = dsum; }
+        __syncthreads();
+        if (t0 + 32 < T) {
+            tq.load(base, C3, t0 + 32, T);
+            tg.load(gbase, C, t0 + 32, T);
+            load_rows(t0 + 32);
+        }
+        if (t0 < k0) continue;                                    // the second wave starts a block later
+        f32x16 p = f32_scores<HD>(sq, mk, lane), ds = f32_scores<HD>(sg, mv, lane);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int row = (r >> 2) * 8 + 4 * half + (r & 3);
+            const bool out_of_it = (t0 == k0 && row < (lane & 31)) || t0 + row >= T;
+            p[r] = out_of_it ? 0.f : expf(p[r] * scale - sl[row]);
+            ds[r] = out_of_it ? 0.f : p[r] * (ds[r] - sd[row]) * scale;
+        }
+        f32_accumulate<HD>(dv, sg, p, lane);
+        f32_accumulate<HD>(dk, sq, ds, lane);
+    }
+    if (k < T) {
+        float* row = dqkv + ((size_t)b * T + k) * C3 + h * HD;
+        f32_store<HD>(row + C, dk, 1.0f, half);
+        f32_store<HD>(row + 2 * C, dv, 1.0f, half);
+    }
+}
+
+template <class F>
+bool with_f32_head(int hs, F f) {
+    switch (hs) {
+        case 32: f(std::integral_constant<int, 32>{}); return true;
+        case 64: f(std::integral_constant<int, 64>{}); return true;
+        case 96: f(std::integral_constant<int, 96>{}); return true;
+        case 128: f(std::integral_constant<int, 128>{}); return true;
+        default: return false;
+    }
+}
+bool f32_aligned(const void* a, const void* b, const void* c, const void* d) {
+    return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c | (uintptr_t)d) % 16) == 0;
+}
+#endif
+
 void launch_forward_rows(floatX* out, float* stats, const floatX* qkv, int B, int T, int NH, int hs, int t0, hipStream_t st) {
+#if defined(LLMK_FP32)
+    if (t0 % 32 == 0 && B * NH <= 65535 && f32_aligned(out, qkv, nullptr, nullptr) && with_f32_head(hs, [&](auto hd) {
+            att_forward_f32_kernel<decltype(hd)::value><<<dim3(CEIL_DIV(T - t0, F_ROWS), B * NH), F_THREADS, 0, st>>>(out, stats, qkv, T, NH, t0);
+        })) return;
+#endif
     const unsigned blocks = (unsigned)CEIL_DIV((size_t)B * NH * (T - t0), (size_t)4);
     if (hs <= 64) att_forward_rows_kernel<1><<<blocks, 256, 0, st>>>(out, stats, qkv, B, T, NH, hs, t0);
     else att_forward_rows_kernel<2><<<blocks, 256, 0, st>>>(out, stats, qkv, B, T, NH, hs, t0);
 }
 void launch_backward_rows(floatX* dqkv, const floatX* dout, const floatX* qkv, const floatX* o, const float* stats, int B,
                           int T, int NH, int hs, hipStream_t st) {
+#if defined(LLMK_FP32)
+    if (B * NH <= 65535 && f32_aligned(dqkv, dout, qkv, o) && with_f32_head(hs, [&](auto hd) {
+            const dim3 grid(CEIL_DIV(T, F_ROWS), B * NH);
+            att_backward_dq_f32_kernel<decltype(hd)::value><<<grid, F_THREADS, 0, st>>>(dqkv, dout, qkv, o, stats, T, NH);
+            att_backward_dkdv_f32_kernel<decltype(hd)::value><<<grid, F_THREADS, 0, st>>>(dqkv, dout, qkv, o, stats, T, NH);
+        })) return;
+#endif
     const unsigned blocks = (unsigned)CEIL_DIV((size_t)B * NH * T, (size_t)4);
     if (hs <= 64) {
         att_backward_dq_rows_kernel<1><<<blocks, 256, 0, st>>>(dqkv, dout, qkv, o, stats, B, T, NH, hs);

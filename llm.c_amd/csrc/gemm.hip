@@ -72,6 +72,14 @@ __device__ __forceinline__ void epilogue_store(const GemmArgs& g, int m, int n, 
     }
 }
 
+// 16-byte rows and pointers, outputs in groups of eight columns, an 8-byte aligned bias: what the direct-to-LDS kernels ask of all operands
+bool operands_ok(const GemmArgs& g) {
+    auto al = [](const void* p, uintptr_t a) { return ((uintptr_t)p % a) == 0; };
+    constexpr int CE = 16 / (int)sizeof(floatX);
+    return g.lda % CE == 0 && g.ldb % CE == 0 && g.ldc % 8 == 0 && g.N % 8 == 0 && al(g.A, 16) && al(g.B, 16) && al(g.C, 16) &&
+           (!g.bias || al(g.bias, 8)) && (!g.aux || al(g.aux, 16));
+}
+
 #if !defined(LLMK_FP32)
 // =============================================================================================
 // bf16 MFMA kernel
@@ -266,11 +274,6 @@ constexpr int BIG_TILE = 256, SMALL_TILE = 128, K_STEP = 64;
 
 // Persistent direct-to-LDS kernel (gemm_pipelined.hpp). Preconditions: K and the per-split K multiples of 32,
 // leading dimensions and N multiples of 8, 16-byte aligned operands, 8-byte aligned bias.
-bool operands_ok(const GemmArgs& g) {
-    auto al = [](const void* p, uintptr_t a) { return ((uintptr_t)p % a) == 0; };
-    return g.lda % 8 == 0 && g.ldb % 8 == 0 && g.ldc % 8 == 0 && g.N % 8 == 0 && al(g.A, 16) && al(g.B, 16) && al(g.C, 16) &&
-           (!g.bias || al(g.bias, 8)) && (!g.aux || al(g.aux, 16));
-}
 bool pipelined_ok(const GemmArgs& g) { return g.K % KGRAN == 0 && g.k_per_split % KGRAN == 0 && operands_ok(g); }
 // The pipelined kernel's += epilogue spills registers (it holds the old values of a whole tile); with it available,
 // a single "split" written as fp32 partials and folded in by the reduce pass is 30 % faster than accumulating in place.
@@ -306,19 +309,6 @@ void launch_best(const GemmArgs& g, int splits, bool big, hipStream_t st) {
     if (pipelined_ok(g)) launch_pipelined<A_T, B_T, EPI>(g, splits, big, st);
     else launch_gemm<A_T, B_T, EPI>(g, splits, big, st);
 }
-constexpr int DINP_MAX_SPLITS = 32, DWEIGHT_MAX_SPLITS = 16;
-// forward: K in one piece, so that a row's sums are taken in one order at every batch size (and no scratch is needed)
-template <int EPI>
-bool launch_forward(const GemmArgs& g, hipStream_t st) {
-    constexpr bool SMALL_TILES = EPI == EPI_BIAS || EPI == EPI_STORE || EPI == EPI_BIAS_GELU;
-    if (!pipelined_ok(g)) return false;
-    const GemmPlan plan = plan_gemm(0, g.M, g.N, g.K, 1, SMALL_TILES, 0, llmk::device_info().num_cu);
-    if (plan.kernel >= 0) launch_ring(plan, g, false, false, EPI, nullptr, st);
-    else if constexpr (SMALL_TILES) launch_pipelined<false, false, EPI>(g, 1, plan.kernel == PERSISTENT_BIG, st);
-    else launch_pipelined_cfg<256, 256, 2, 4, false, false, EPI>(g, 1, st);
-    return true;
-}
-
 #else
 // =============================================================================================
 // fp32 MFMA kernel (parity mode): 128x128 tile, K step 16, 4 waves of 64x64
@@ -447,6 +437,25 @@ void launch_best(const GemmArgs& g, int splits, bool big, hipStream_t st) { laun
 bool tn_partial_always(const GemmArgs&) { return false; }
 #endif
 
+constexpr int DINP_MAX_SPLITS = 32, DWEIGHT_MAX_SPLITS = 16;
+// K of the operands whose rows it runs along: a whole number of stages
+bool ring_k_ok(const GemmArgs& g) { return g.K % RING_K == 0 && g.K > 0 && operands_ok(g); }
+// forward: K in one piece, so that a row's sums are taken in one order at every batch size (and no scratch is needed)
+template <int EPI>
+bool launch_forward(const GemmArgs& g, hipStream_t st) {
+    constexpr bool SMALL_TILES = EPI == EPI_BIAS || EPI == EPI_STORE || EPI == EPI_BIAS_GELU;
+    if (!ring_k_ok(g)) return false;
+    const GemmPlan plan = plan_gemm(0, g.M, g.N, g.K, 1, SMALL_TILES, 0, llmk::device_info().num_cu);
+    if (plan.kernel >= 0) { launch_ring(plan, g, false, false, EPI, nullptr, st); return true; }
+#if defined(LLMK_FP32)
+    return false;
+#else
+    if constexpr (SMALL_TILES) launch_pipelined<false, false, EPI>(g, 1, plan.kernel == PERSISTENT_BIG, st);
+    else launch_pipelined_cfg<256, 256, 2, 4, false, false, EPI>(g, 1, st);
+    return true;
+#endif
+}
+
 enum { SKR_STORE = 0, SKR_ACCUM = 1, SKR_DGELU = 2, SKR_DGELU_D = 3 };    // (the last two: times gelu'(aux), times aux)
 // C[m][n] (+)= sum over splits of partial[s][m][n], in split order. Workgroups past the ones that cover C add up the
 // row sums of EPI_PARTIAL_ROWSUM: rowvec[m] += sum over parts of rowsum[p][m], 32 rows per workgroup, 8 groups of lanes
@@ -502,7 +511,6 @@ splitk_reduce_kernel(floatX* __restrict__ C, const floatX* __restrict__ aux, con
 // instead, each workgroup at its own K offset, left every panel to be streamed once per tile: slower than the equal
 // splits). Partial slot = rank of the piece along K, so the sum order is fixed.
 constexpr int SK_MIN_BLOCKS = 4;
-int g_sk_mode = -1;                  // llmk_matmul_backward_split_mode
 struct SkPlan {
     int slots = 0;                   // pieces per tile
     int long_blocks = 0;             // K blocks of the long piece
@@ -549,21 +557,20 @@ int tn_equal_splits(int M, size_t tiles, int num_cu, double* cost_out) {
     return CEIL_DIV(ksteps, CEIL_DIV(ksteps, splits));
 }
 
-#if !defined(LLMK_FP32)
 // The weight gradient dW[OC][C] over M rows: the persistent kernel and its pass over partial products against the ring
 // kernels, which also take a number of rows that is not a multiple of 64
 GemmPlan dweight_plan(int M, int C, int OC, int num_cu) {
     const size_t big_tiles = (size_t)CEIL_DIV(OC, BIG_TILE) * CEIL_DIV(C, BIG_TILE);
     const bool big = big_tiles >= 8;
     double us = std::numeric_limits<double>::infinity();
-    if (M % K_STEP == 0) {
+    if (sizeof(floatX) == 2 && M % K_STEP == 0) {
         const size_t tiles = big ? big_tiles : (size_t)CEIL_DIV(OC, SMALL_TILE) * CEIL_DIV(C, SMALL_TILE);
         us = persistent_tn_us(OC, C, M, tn_equal_splits(M, tiles, num_cu, nullptr), big, num_cu);
     }
     return plan_gemm(2, OC, C, M, DWEIGHT_MAX_SPLITS, false, us, num_cu);
 }
-#endif
 
+int g_split_mode = -1;                // llmk_matmul_backward_split_mode
 // what the last weight-gradient GEMM did with K: 0 = not cut, 1 = equal splits, 2 = one long + short pieces
 int g_last_split_kind = 0, g_last_split_pieces = 0;
 
@@ -739,26 +746,18 @@ void llmk_matmul_forward(void* out, const void* inp, const void* weight, const v
     if (pre_gelu && gelu_fusion >= 3) {
         // pre_gelu receives gelu'(pre-activation): in the epilogue of the direct-to-LDS kernels, else by a pass of its own
         g.C = (floatX*)out; g.aux = (floatX*)pre_gelu;
-#if !defined(LLMK_FP32)
         if (launch_forward<EPI_BIAS_GELU_D>(g, st)) return;
-#endif
         g.C = (floatX*)pre_gelu; g.aux = nullptr;
         launch_best<false, false, EPI_BIAS>(g, 1, big, st);
         if (prof.on) { llmk::prof_end(st); prof.on = false; }
         llmk_gelu_forward_keep_grad(out, pre_gelu, M * OC, stream);
     } else if (pre_gelu && gelu_fusion >= 1) {
         g.C = (floatX*)out; g.aux = (floatX*)pre_gelu;
-#if !defined(LLMK_FP32)
         if (launch_forward<EPI_BIAS_GELU>(g, st)) return;
-#endif
         launch_best<false, false, EPI_BIAS_GELU>(g, 1, big, st);
     } else {
         g.C = (floatX*)(pre_gelu ? pre_gelu : out);
-#if !defined(LLMK_FP32)
         const bool done = bias ? launch_forward<EPI_BIAS>(g, st) : launch_forward<EPI_STORE>(g, st);   // the LM head: no bias to fetch, no window to keep for it
-#else
-        const bool done = false;
-#endif
         if (done) {
         } else if (bias) launch_best<false, false, EPI_BIAS>(g, 1, big, st);
         else launch_best<false, false, EPI_STORE>(g, 1, big, st);
@@ -789,7 +788,7 @@ size_t llmk_matmul_backward_bias_scratch_floats(int OC) { return (size_t)bias_gr
 
 void llmk_matmul_backward_split_mode(int mode) {
 #if !defined(LLMK_FP32)
-    g_sk_mode = mode < 0 ? -1 : mode > 0 ? 1 : 0;
+    g_split_mode = mode < 0 ? -1 : mode > 0 ? 1 : 0;
 #else
     (void)mode;                          // the fp32 library has one weight-gradient path
 #endif
@@ -812,10 +811,12 @@ size_t llmk_matmul_backward_workspace_bytes(int B, int T, int C, int OC) {
         const SkPlan plan = sk_build(CEIL_DIV(OC, BIG_TILE), CEIL_DIV(C, BIG_TILE), M / K_STEP, num_cu & ~7, 800.0 / (double)M);
         if (plan.valid) pieces = max(pieces, plan.slots);
     }
-    pieces = max(pieces, dweight_plan(M, C, OC, num_cu).splits);
-    const int dinp_pieces = plan_gemm(1, M, C, OC, DINP_MAX_SPLITS, true, 0, num_cu).splits;
-    if (dinp_pieces > 1) dinp = (size_t)M * C * dinp_pieces * sizeof(float);
 #endif
+    pieces = max(pieces, dweight_plan(M, C, OC, num_cu).splits);
+    for (const bool small_tiles : {false, true}) {                // (with GELU backward in the epilogue, and without)
+        const int dinp_pieces = plan_gemm(1, M, C, OC, DINP_MAX_SPLITS, small_tiles, 0, num_cu).splits;
+        if (dinp_pieces > 1) dinp = max(dinp, (size_t)M * C * dinp_pieces * sizeof(float));
+    }
     return max(dinp, ((size_t)OC * C + (size_t)OC * 4) * pieces * sizeof(float));     // partial products + the bias gradient's row sums
 }
 
@@ -863,21 +864,23 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
     // it adds up the rows of that operand on the side (EPI_PARTIAL_ROWSUM), which is the bias gradient without another
     // pass over dout. Same preconditions as that kernel; otherwise the streaming reduction in (1).
     bool dbias_in_gemm = false;
-#if !defined(LLMK_FP32)
     GemmPlan dw_plan;                    // of the ring kernels, or left at the persistent one's
     {
         GemmArgs t{};
         t.A = (const floatX*)dout; t.B = (const floatX*)inp; t.C = (floatX*)dweight;
-        t.M = OC; t.N = C; t.K = M; t.lda = OC; t.ldb = C; t.ldc = C; t.k_per_split = KGRAN;
-        if (operands_ok(t) && g_sk_mode < 0) dw_plan = dweight_plan(M, C, OC, num_cu);
-        dbias_in_gemm = dbias && (dw_plan.kernel >= 0 || pipelined_ok(t));
-        LLMK_REQUIRE(!dbias || pipelined_ok(t) || dbias_buffer != nullptr, "matmul_backward: dbias_buffer is required when dbias is given");
-    }
+        t.M = OC; t.N = C; t.K = M; t.lda = OC; t.ldb = C; t.ldc = C; t.k_per_split = K_STEP;
+        if (operands_ok(t) && g_split_mode < 0) dw_plan = dweight_plan(M, C, OC, num_cu);
+#if defined(LLMK_FP32)
+        const bool persistent = false;
+#else
+        const bool persistent = pipelined_ok(t);
 #endif
+        dbias_in_gemm = dbias && (dw_plan.kernel >= 0 || persistent);
+        LLMK_REQUIRE(!dbias || persistent || dbias_buffer != nullptr, "matmul_backward: dbias_buffer is required when dbias is given");
+    }
 
     // (1) dbias += column sums of dout
     if (dbias && !dbias_in_gemm) {
-        LLMK_REQUIRE(dbias_buffer != nullptr, "matmul_backward: dbias_buffer is required when dbias is given");
         const int ny = bias_grad_ny(OC);
         llmk::ProfScope prof("bias_grad", 0, (double)M * OC * sizeof(floatX), st);
         bias_grad_kernel<false><<<dim3(CEIL_DIV(OC, BG_COLV * VN), ny), 256, 0, st>>>(dbias_buffer, (floatX*)dout, nullptr, M, OC);
@@ -894,24 +897,23 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
         g.k_per_split = CEIL_DIV(OC, K_STEP) * K_STEP;
         const bool big = (size_t)CEIL_DIV(M, BIG_TILE) * CEIL_DIV(C, BIG_TILE) >= (size_t)num_cu;
         const bool stored_grad = pre_gelu && gelu_fusion >= 3;   // pre_gelu holds gelu'(pre-activation), see llmk_matmul_forward
+        // gelu' goes into the epilogue of the direct-to-LDS kernels; the bias gradient of the layer below then comes out of
+        // its weight-gradient GEMM, and no elementwise pass over (B,T,4C) is left
+        const bool ring = ring_k_ok(g);
 #if defined(LLMK_FP32)
-        const bool fused = pre_gelu && gelu_fusion >= 2 && !stored_grad;
+        const bool fused = pre_gelu && gelu_fusion >= 2 && (!stored_grad || (ring && aligned16(pre_gelu)));
+        const bool fused_in_ring = fused && aligned16(pre_gelu);
 #else
-        // bf16: gelu' goes into the epilogue of the direct-to-LDS kernels; the bias gradient of the layer
-        // below then comes out of its weight-gradient GEMM, and no elementwise pass over (B,T,4C) is left
         const bool fused = pre_gelu && gelu_fusion >= 2 && aligned16(pre_gelu) && pipelined_ok(g);
-        GemmPlan plan;
-        if (pipelined_ok(g)) plan = plan_gemm(1, M, C, OC, DINP_MAX_SPLITS, !fused, 0, num_cu);
+        const bool fused_in_ring = fused;
 #endif
+        GemmPlan plan;
+        if (ring && fused == fused_in_ring) plan = plan_gemm(1, M, C, OC, DINP_MAX_SPLITS, !fused, 0, num_cu);
         {
             // with GELU backward in the epilogue the kernel also reads the (M, C) pre-activations
             llmk::ProfScope prof(fused ? "gemm_nn_dgelu" : "gemm_nn", 2.0 * M * (double)OC * C,
                                  ((double)M * OC + (double)OC * C + (fused ? 2.0 : 1.0) * M * C) * sizeof(floatX), st);
             if (fused) g.aux = (floatX*)pre_gelu;
-#if defined(LLMK_FP32)
-            if (fused) launch_best<false, true, EPI_DGELU>(g, 1, big, st);
-            else launch_best<false, true, EPI_STORE>(g, 1, big, st);
-#else
             if (plan.kernel >= 0 && plan.splits > 1) {
                 const size_t mn = (size_t)M * C;
                 g.partial = (float*)llmk::workspace(mn * plan.splits * sizeof(float));
@@ -927,12 +929,15 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
             } else if (plan.kernel >= 0) {
                 launch_ring(plan, g, false, true, !fused ? EPI_STORE : stored_grad ? EPI_DGELU_D : EPI_DGELU, nullptr, st);
             } else if (fused) {
+#if defined(LLMK_FP32)
+                launch_best<false, true, EPI_DGELU>(g, 1, big, st);
+#else
                 if (stored_grad) launch_pipelined_cfg<256, 256, 2, 4, false, true, EPI_DGELU_D>(g, 1, st);
                 else launch_pipelined_cfg<256, 256, 2, 4, false, true, EPI_DGELU>(g, 1, st);
-            } else {
-                launch_best<false, true, EPI_STORE>(g, 1, pipelined_ok(g) ? plan.kernel == PERSISTENT_BIG : big, st);
-            }
 #endif
+            } else {
+                launch_best<false, true, EPI_STORE>(g, 1, ring ? plan.kernel == PERSISTENT_BIG : big, st);
+            }
         }
         if (pre_gelu && !fused) {
             if (stored_grad) llmk_gelu_backward_from_grad(dinp, pre_gelu, M * C, stream);
@@ -953,7 +958,6 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
         const int splits = tn_equal_splits(M, tiles, num_cu, &best_uniform);
         g.k_per_split = CEIL_DIV(CEIL_DIV(M, K_STEP), splits) * K_STEP;
         const double tn_bytes = ((double)M * OC + (double)M * C + 2.0 * OC * C) * sizeof(floatX);
-#if !defined(LLMK_FP32)
         if (dw_plan.kernel >= 0) {
             const int pieces = dw_plan.splits;
             const size_t mn = (size_t)OC * C;
@@ -972,17 +976,16 @@ void llmk_matmul_backward(void* dinp, void* dweight, void* dbias, const void* do
             LAUNCH_CHECK();
             return;
         }
-#endif
         if (splits == 1 && !tn_partial_always(g)) {
             LLMK_REQUIRE(!dbias_in_gemm, "matmul_backward: bias gradient was left to a kernel that is not being run");
             llmk::ProfScope prof("gemm_tn", 2.0 * M * (double)OC * C, tn_bytes, st);
             launch_best<true, true, EPI_ACCUM>(g, 1, big, st);
             g_last_split_kind = 0; g_last_split_pieces = 1;
 #if !defined(LLMK_FP32)
-        } else if (const SkPlan plan = (big && M % K_STEP == 0 && pipelined_ok(g) && (!dbias || dbias_in_gemm) && g_sk_mode != 0)
+        } else if (const SkPlan plan = (big && M % K_STEP == 0 && pipelined_ok(g) && (!dbias || dbias_in_gemm) && g_split_mode != 0)
                                            ? sk_build(CEIL_DIV(OC, BIG_TILE), CEIL_DIV(C, BIG_TILE), M / K_STEP, num_cu & ~7, 800.0 / (double)M)
                                            : SkPlan();
-                   plan.valid && (g_sk_mode == 1 || plan.cost < 0.98 * best_uniform)) {
+                   plan.valid && (g_split_mode == 1 || plan.cost < 0.98 * best_uniform)) {
             // one long and s - 1 short pieces per tile (see sk_build)
             const size_t mn = (size_t)OC * C;
             const int parts = 4, slots = plan.slots, G = num_cu & ~7;

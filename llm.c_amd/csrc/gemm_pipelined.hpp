@@ -76,6 +76,48 @@ struct GemmArgs {
 };
 constexpr int SK_MAX_ITEMS = 8;         // most short pieces one workgroup takes
 
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): loops whose index has to be a constant expression
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
+
+// wait until at most N of this wave's vector-memory operations are outstanding (gfx9 encoding, other counters untouched)
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+// Registers loaded by inline asm, whose completion the compiler does not track: after the wait for them they pass through
+// here, so that nothing that reads them can move above it
+template <typename V>
+__device__ __forceinline__ void tie4(V& a, V& b, V& c, V& d) { asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d)); }
+
+// Workgroup barrier WITHOUT the memory fence of __syncthreads(): the fence would wait for every outstanding
+// direct-to-LDS load (vmcnt(0)) and serialize the pipeline. Visibility of the K block that is about to be
+// read is established by the explicit vmcnt wait each wave does before arriving here.
+__device__ __forceinline__ void barrier_no_fence() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// tile id -> tile coordinates; consecutive ids walk a group of TILE_GROUP rows of tiles column by column. The 32 CUs
+// of an XCD then hold 4 row panels and 8 column panels at a time; groups of 8 and 16 measured 0.3 % and 1.5 % slower
+// on the whole training step, groups of 2 the same, single rows 0.6 % slower.
+#ifndef LLMK_TILE_GROUP
+#define LLMK_TILE_GROUP 4
+#endif
+constexpr int TILE_GROUP = LLMK_TILE_GROUP;
+__device__ __forceinline__ void tile_of(int t, int tiles_m, int tiles_n, int& tm, int& tn) {
+    const int per_group = TILE_GROUP * tiles_n;
+    const int group = t / per_group;
+    const int first_m = group * TILE_GROUP;
+    const int gsz = min(tiles_m - first_m, TILE_GROUP);
+    const int in_group = t - group * per_group;
+    tm = first_m + in_group % gsz;
+    tn = in_group / gsz;
+}
+
 #if !defined(LLMK_FP32)
 
 #ifndef LLMK_TR_ASM_BOTH
@@ -116,31 +158,6 @@ constexpr int smem_bytes(int bm, int bn, int nw) { return STAGES * (bm + bn) * P
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): loops whose index has to be a constant expression
-template <class F, int... I>
-__device__ __forceinline__ void static_for_impl(F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
-
-// wait until at most N of this wave's vector-memory operations are outstanding (gfx9 encoding, other counters untouched)
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-// Registers loaded by inline asm, whose completion the compiler does not track: after the wait for them they pass through
-// here, so that nothing that reads them can move above it
-template <typename V>
-__device__ __forceinline__ void tie4(V& a, V& b, V& c, V& d) { asm volatile("" : "+v"(a), "+v"(b), "+v"(c), "+v"(d)); }
-
-// Workgroup barrier WITHOUT the memory fence of __syncthreads(): the fence would wait for every outstanding
-// direct-to-LDS load (vmcnt(0)) and serialize the pipeline. Visibility of the K block that is about to be
-// read is established by the explicit vmcnt wait each wave does before arriving here.
-__device__ __forceinline__ void barrier_no_fence() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // Output stores are non-temporal: a tile's output is not read again by this kernel, and a store that allocates in
 // L2 is acknowledged late enough (the waves count stores and loads with one counter) to hold up the next tile's loads.
 template <typename T>
@@ -160,23 +177,6 @@ __device__ __forceinline__ s16x4 ds_read_tr16(unsigned addr) {
     s16x4 v;
     asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
     return v;
-}
-
-// tile id -> tile coordinates; consecutive ids walk a group of TILE_GROUP rows of tiles column by column. The 32 CUs
-// of an XCD then hold 4 row panels and 8 column panels at a time; groups of 8 and 16 measured 0.3 % and 1.5 % slower
-// on the whole training step, groups of 2 the same, single rows 0.6 % slower.
-#ifndef LLMK_TILE_GROUP
-#define LLMK_TILE_GROUP 4
-#endif
-constexpr int TILE_GROUP = LLMK_TILE_GROUP;
-__device__ __forceinline__ void tile_of(int t, int tiles_m, int tiles_n, int& tm, int& tn) {
-    const int per_group = TILE_GROUP * tiles_n;
-    const int group = t / per_group;
-    const int first_m = group * TILE_GROUP;
-    const int gsz = min(tiles_m - first_m, TILE_GROUP);
-    const int in_group = t - group * per_group;
-    tm = first_m + in_group % gsz;
-    tn = in_group / gsz;
 }
 
 template <int BM, int BN, int WGM, int WGN, bool A_T, bool B_T, int EPI>

@@ -3,16 +3,16 @@
 #include "gelu.hpp"
 #include "gemm_ring.hpp"
 #include <algorithm>
+#include <limits>
 #include "../../include/llmk.h"
 
-#if !defined(LLMK_FP32)
 namespace gemmk {
 namespace {
 
-// What a stage past the end of K is read from (both operands K-major, K not a multiple of 64)
+// What a stage past the end of K is read from (both operands K-major, K not a multiple of RING_K)
 __device__ const u32x4 g_zero_chunk = {0, 0, 0, 0};
 
-// One output tile (and one piece of K) per workgroup; K in stages of 64 through a ring of NST LDS buffers, NST - 1 of them
+// One output tile (and one piece of K) per workgroup; K in stages of RING_K through a ring of NST LDS buffers, NST - 1 of them
 // in flight. A launch of few tiles has nothing to hide memory latency behind but its own lookahead: with the two buffers of
 // the persistent kernel a stage costs a trip to HBM. Operand layouts, swizzles, fragment reads and the order of every sum are the
 // persistent kernel's, so that a forward pass has the same bits whichever of the two ran it. The finished tile goes through
@@ -23,13 +23,22 @@ __device__ const u32x4 g_zero_chunk = {0, 0, 0, 0};
 // Measured, weights from HBM, us, the persistent kernel's better tile against this: 256 x 768 over K = 3072 29.6 / 15.0 (one
 // piece), 9.9 (four, with the pass over the partials), over K = 50304 613 / 42; 4096 x 2048 over 8192 156 / 123; 3000 x 1536 over
 // 6144 120 / 82; dweight 3072 x 768 over 256 rows 19.7 / 7.1, 4608 x 1536 over 3000 rows (no persistent kernel) 83 / 52.
+// The fp32 library has the same kernel with the fp32 matrix instruction, 16 of which make a stage of 32: the matrix cores bound
+// it (2048 x 50304 over 768: 119 TFLOP/s of 157) as soon as every CU has a tile, so what counts is tiles small enough for that.
+constexpr int CE = 16 / (int)sizeof(floatX);     // elements of a 16-byte chunk
+#if defined(LLMK_FP32)
+typedef f32x4 frag_t;                            // eight of K: lane half h holds 4 h .. 4 h + 3
+#else
+typedef bf16x8 frag_t;                           // sixteen of K
+#endif
+
 template <int BM, int BN, int WGM, int WGN, int NST, bool A_T, bool B_T>
 __global__ void __launch_bounds__(WGM * WGN * 64)
 gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int NW = WGM * WGN, NT = NW * 64;
     constexpr int WTM = BM / WGM, WTN = BN / WGN, TM = WTM / 32, TN = WTN / 32;
-    constexpr int A_STAGE = BM * PBK * 2, B_STAGE = BN * PBK * 2, STAGE = A_STAGE + B_STAGE;
+    constexpr int A_STAGE = BM * 128, B_STAGE = BN * 128, STAGE = A_STAGE + B_STAGE, X = (int)sizeof(floatX);
     constexpr int A_CHUNKS = A_STAGE / 1024, B_CHUNKS = B_STAGE / 1024, CPW = (A_CHUNKS + B_CHUNKS) / NW;
     static_assert(A_CHUNKS % NW == 0 && B_CHUNKS % NW == 0, "each load slot of a wave is all-A or all-B");
     static_assert(NST >= 2 && (NST - 2) * CPW <= 63, "vmcnt is a 6-bit counter");
@@ -52,18 +61,18 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
     const int split = id / num_tiles;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int kbeg = split * g.k_per_split, kend = min(g.K, kbeg + g.k_per_split);
-    const int nst = CEIL_DIV(kend - kbeg, PBK);
-    const int tail = K_TAIL && (kend - kbeg) % PBK ? nst - 1 : -1;      // the stage that reaches past K
+    const int nst = CEIL_DIV(kend - kbeg, RING_K);
+    const int tail = K_TAIL && (kend - kbeg) % RING_K ? nst - 1 : -1;      // the stage that reaches past K
 
     typedef __attribute__((address_space(3))) const char* lds_cptr;
     const unsigned lds0 = (unsigned)(size_t)(lds_cptr)lds;
     const char* base_a = reinterpret_cast<const char*>(A_T ? g.A + (size_t)kbeg * g.lda + m0 : g.A + (size_t)m0 * g.lda + kbeg);
     const char* base_b = reinterpret_cast<const char*>(B_T ? g.B + (size_t)kbeg * g.ldb + n0 : g.B + (size_t)n0 * g.ldb + kbeg);
-    const size_t step_a = (A_T ? (size_t)PBK * g.lda : (size_t)PBK) * sizeof(floatX);
-    const size_t step_b = (B_T ? (size_t)PBK * g.ldb : (size_t)PBK) * sizeof(floatX);
-    // K-major tiles [k][rows]: which 16-byte chunk of row k a lane fetches, so that the transposing reads of four
-    // consecutive k meet no bank twice
-    auto swz_t = [](int rows, int k) { return rows >= 128 ? 4 * (k & 3) : rows == 64 ? 4 * ((k >> 1) & 1) : 0; };
+    const size_t step_a = (A_T ? (size_t)RING_K * g.lda : (size_t)RING_K) * X;
+    const size_t step_b = (B_T ? (size_t)RING_K * g.ldb : (size_t)RING_K) * X;
+    // K-major tiles [k][rows]: which 16-byte chunk of row k a lane fetches, so that the reads - of four consecutive k by the
+    // transposing read, of k and k + 4 by the two half-waves in fp32 - meet no bank twice
+    auto swz_t = [](int rows, int k) { return X == 4 ? 8 * ((k >> 2) & 1) : rows >= 128 ? 4 * (k & 3) : 4 * ((k >> 1) & 1); };
     unsigned voff[CPW];
     int krow_of[K_TAIL ? CPW : 1];
 #pragma unroll
@@ -73,10 +82,10 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
         const int ld = isA ? g.lda : g.ldb, r0 = isA ? m0 : n0, rmax = isA ? g.M : g.N, R = isA ? BM : BN;
         if (!(isA ? A_T : B_T)) {
             const int row = cc * 8 + (lane >> 3), c = (lane & 7) ^ ((row >> 1) & 7);
-            voff[i] = ((unsigned)min(row, rmax - 1 - r0) * (unsigned)ld + c * 8) * (unsigned)sizeof(floatX);
+            voff[i] = ((unsigned)min(row, rmax - 1 - r0) * (unsigned)ld + c * CE) * (unsigned)X;
         } else {
-            const int byte = cc * 1024 + lane * 16, krow = byte / (R * 2), cn = ((byte % (R * 2)) >> 4) ^ swz_t(R, krow);
-            voff[i] = ((unsigned)krow * (unsigned)ld + (r0 + cn * 8 < rmax ? cn * 8 : 0)) * (unsigned)sizeof(floatX);
+            const int byte = cc * 1024 + lane * 16, krow = byte / (R * X), cn = ((byte % (R * X)) >> 4) ^ swz_t(R, krow);
+            voff[i] = ((unsigned)krow * (unsigned)ld + (r0 + cn * CE < rmax ? cn * CE : 0)) * (unsigned)X;
             if (K_TAIL) krow_of[i] = krow;
         }
     }
@@ -89,7 +98,7 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
         if (K_TAIL && st == tail) {                               // rows past K are zeros
 #pragma unroll
             for (int i = 0; i < CPW; i++) {
-                const bool in = kbeg + st * PBK + krow_of[K_TAIL ? i : 0] < kend;
+                const bool in = kbeg + st * RING_K + krow_of[K_TAIL ? i : 0] < kend;
                 const unsigned long long p = in ? (i * NW < A_CHUNKS ? pa : pb) + voff[i] : (unsigned long long)(size_t)&g_zero_chunk;
                 asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(stage + (wave + i * NW) * 1024), "v"(p) : "memory");
             }
@@ -107,6 +116,10 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
             const int row = row0 + idx;
             return region + row * 128 + ((((row >> 1) & 7) ^ half) << 4);
         }
+        if (X == 4) {                                             // row 4 half + e of eight, column idx
+            const int col = row0 + idx;
+            return region + 4 * half * (rows * 4) + ((col >> 2) ^ swz_t(rows, 4 * half)) * 16 + (col & 3) * 4;
+        }
         const int s16 = lane & 15, grp = lane >> 4;
         const int krow = 8 * (grp >> 1) + (s16 >> 2), col = row0 + (grp & 1) * 16 + 4 * (s16 & 3);
         return region + krow * (rows * 2) + ((col >> 3) ^ swz_t(rows, krow)) * 16 + (col & 7) * 2;
@@ -116,16 +129,23 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
     for (int i = 0; i < TM; i++) abase[i] = lds0 + frag_base(A_T, 0, BM, wm * WTM + i * 32);
 #pragma unroll
     for (int j = 0; j < TN; j++) bbase[j] = lds0 + frag_base(B_T, A_STAGE, BN, wn * WTN + j * 32);
-    auto frag = [&](bool trans, unsigned base, unsigned buf, int s, int rows) -> bf16x8 {
+    auto frag = [&](bool trans, unsigned base, unsigned buf, int s, int rows) -> frag_t {
         if (!trans)
-            return *reinterpret_cast<const __attribute__((address_space(3))) bf16x8*>((size_t)((base ^ (unsigned)(s << 5)) + buf));
+            return *reinterpret_cast<const __attribute__((address_space(3))) frag_t*>((size_t)((base ^ (unsigned)(s << 5)) + buf));
+#if defined(LLMK_FP32)
+        frag_t v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = *reinterpret_cast<const __attribute__((address_space(3))) float*>((size_t)(base + buf + (8 * s + e) * rows * 4));
+        return v;
+#else
         typedef s16x4 __attribute__((address_space(3))) * lp;
         union { struct { s16x4 a, b; } p; bf16x8 v; } u;
         u.p.a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(size_t)(base + buf + s * 16 * rows * 2));
         u.p.b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(size_t)(base + buf + (s * 16 + 4) * rows * 2));
         return u.v;
+#endif
     };
-    auto read_frags = [&](int b, int s, bf16x8 (&fa)[TM], bf16x8 (&fb)[TN]) {
+    auto read_frags = [&](int b, int s, frag_t (&fa)[TM], frag_t (&fb)[TN]) {
         const unsigned buf = (unsigned)b * STAGE;
 #pragma unroll
         for (int i = 0; i < TM; i++) fa[i] = frag(A_T, abase[i], buf, s, BM);
@@ -144,13 +164,26 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
     float rsum[A_T ? TM : 1];
 #pragma unroll
     for (int i = 0; i < (A_T ? TM : 1); i++) rsum[i] = 0.f;
-    auto mma = [&](const bf16x8 (&fa)[TM], const bf16x8 (&fb)[TN], int s) {
+    auto mma = [&](const frag_t (&fa)[TM], const frag_t (&fb)[TN], int s) {
+#if defined(LLMK_FP32)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[j][e], fa[i][e], acc[i][j], 0, 0, 0);
+#else
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+#endif
         if constexpr (A_T) {
             if (rowsum && s % WGN == wn) {
+#if defined(LLMK_FP32)
+#pragma unroll
+                for (int i = 0; i < TM; i++) rsum[i] += (fa[i][0] + fa[i][1]) + (fa[i][2] + fa[i][3]);
+#else
                 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
                 const bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
 #pragma unroll
@@ -160,6 +193,7 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
                         const bf16x2 p = {fa[i][2 * e], fa[i][2 * e + 1]};
                         rsum[i] = __builtin_amdgcn_fdot2_f32_bf16(p, ones, rsum[i], false);
                     }
+#endif
             }
         }
     };
@@ -174,7 +208,7 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
 #pragma unroll
     for (int s = 0; s < NST - 1; s++)
         if (s < nst) issue(s, s);
-    bf16x8 fa0[TM], fb0[TN], fa1[TM], fb1[TN];
+    frag_t fa0[TM], fb0[TN], fa1[TM], fb1[TN];
     wait_stage(0);
     barrier_no_fence();
     if (NST - 1 < nst) issue(NST - 1, NST - 1);
@@ -247,45 +281,60 @@ gemm_ring_kernel(GemmArgs g, int epi, floatX* rowvec) {
             *reinterpret_cast<f32x4*>(p + 4) = *reinterpret_cast<f32x4*>(x + 4);
             continue;
         }
-        union V { u32x4 u; bf16x8 h; };
-        if (g.bias) {                                             // (the callers give one to the epilogues that have one)
-            const bf16x4 b0 = *reinterpret_cast<const bf16x4*>(g.bias + n), b1 = *reinterpret_cast<const bf16x4*>(g.bias + n + 4);
+        // eight columns in storage type: 16 bytes, or 32 in fp32
+        struct alignas(CE == 8 ? 16 : 32) V { floatX h[8]; };
+        auto load8 = [](const floatX* p) {
+            V v;
 #pragma unroll
-            for (int e = 0; e < 4; e++) { x[e] += (float)b0[e]; x[4 + e] += (float)b1[e]; }
+            for (int k = 0; k < 8 / CE; k++) reinterpret_cast<u32x4*>(&v)[k] = reinterpret_cast<const u32x4*>(p)[k];
+            return v;
+        };
+        auto store8 = [](floatX* p, const V& v) {
+#pragma unroll
+            for (int k = 0; k < 8 / CE; k++) reinterpret_cast<u32x4*>(p)[k] = reinterpret_cast<const u32x4*>(&v)[k];
+        };
+        if (g.bias) {                                             // (the callers give one to the epilogues that have one)
+            typedef floatX half_t __attribute__((ext_vector_type(8 / (int)sizeof(floatX))));      // 8 bytes: the alignment asked of a bias
+#pragma unroll
+            for (int k = 0; k < X; k++) {
+                const half_t b = reinterpret_cast<const half_t*>(g.bias + n)[k];
+#pragma unroll
+                for (int e = 0; e < 8 / X; e++) x[8 / X * k + e] += (float)b[e];
+            }
         }
         V y, a;
         if (epi == EPI_ACCUM) {
-            a.u = *reinterpret_cast<const u32x4*>(g.C + o);
+            a = load8(g.C + o);
 #pragma unroll
-            for (int e = 0; e < 8; e++) y.h[e] = (__bf16)((float)a.h[e] + x[e]);
+            for (int e = 0; e < 8; e++) y.h[e] = (floatX)((float)a.h[e] + x[e]);
         } else {
 #pragma unroll
-            for (int e = 0; e < 8; e++) y.h[e] = (__bf16)x[e];
+            for (int e = 0; e < 8; e++) y.h[e] = (floatX)x[e];
             if (epi_gelu_fwd(epi)) {
                 a = y;
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    if (epi == EPI_BIAS_GELU) y.h[e] = (__bf16)gelu_f((float)y.h[e]);
-                    else { float gr; y.h[e] = (__bf16)gelu_with_grad_f((float)y.h[e], gr); a.h[e] = (__bf16)gr; }
+                    if (epi == EPI_BIAS_GELU) y.h[e] = (floatX)gelu_f((float)y.h[e]);
+                    else { float gr; y.h[e] = (floatX)gelu_with_grad_f((float)y.h[e], gr); a.h[e] = (floatX)gr; }
                 }
-                *reinterpret_cast<u32x4*>(g.aux + o) = a.u;
+                store8(g.aux + o, a);
             } else if (epi_reads_aux(epi)) {
-                a.u = *reinterpret_cast<const u32x4*>(g.aux + o);
+                a = load8(g.aux + o);
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
                     const float p = (float)a.h[e], d = (float)y.h[e];
-                    y.h[e] = (__bf16)(epi == EPI_BIAS_RES ? d + p : (epi == EPI_DGELU_D ? p : gelu_grad_f(p)) * d);
+                    y.h[e] = (floatX)(epi == EPI_BIAS_RES ? d + p : (epi == EPI_DGELU_D ? p : gelu_grad_f(p)) * d);
                 }
             }
         }
-        *reinterpret_cast<u32x4*>(g.C + o) = y.u;
+        store8(g.C + o, y);
     }
 #endif
 }
 
 template <int BM, int BN, int WGM, int WGN, int NST, bool A_T, bool B_T>
 void launch_cfg(const GemmArgs& g, int epi, floatX* rowvec, hipStream_t st) {
-    constexpr int SMEM = NST * (BM + BN) * PBK * 2;
+    constexpr int SMEM = NST * (BM + BN) * 128;
     auto kern = gemm_ring_kernel<BM, BN, WGM, WGN, NST, A_T, B_T>;
     static bool attr_set = false;
     if (!attr_set) {
@@ -313,6 +362,15 @@ void launch_layout(int cfg, const GemmArgs& g, int epi, floatX* rowvec, hipStrea
 // (the CUs then share L2 and HBM, and a workgroup its CU's LDS with its neighbours); between, in proportion to the load.
 struct TileCost { int bm, bn, per_cu; double alone, full[3], fixed; };      // full: forward, dinp, dweight
 constexpr int RING_CFGS = 5;
+#if defined(LLMK_FP32)
+constexpr TileCost RING_COST[RING_CFGS] = {
+    {256, 128, 1, 3.75, {3.9, 3.9, 4.1}, 7.0},
+    {128, 128, 2, 1.95, {3.9, 3.9, 4.1}, 6.0},
+    {128, 128, 1, 1.95, {2.0, 2.0, 2.1}, 6.0},
+    {128, 64, 2, 1.0, {1.95, 1.95, 2.05}, 5.0},
+    {64, 64, 3, 0.52, {1.5, 1.5, 1.55}, 4.0},
+};
+#else
 constexpr TileCost RING_COST[RING_CFGS] = {
     {256, 128, 1, 0.75, {0.97, 0.95, 1.12}, 5.0},
     {128, 128, 2, 0.57, {0.96, 1.09, 1.10}, 4.5},
@@ -320,10 +378,11 @@ constexpr TileCost RING_COST[RING_CFGS] = {
     {128, 64, 2, 0.39, {0.62, 0.62, 0.72}, 3.6},
     {64, 64, 3, 0.29, {0.58, 0.58, 0.64}, 2.8},
 };
+#endif
 constexpr TileCost PERSISTENT_COST[2] = {{256, 256, 1, 1.07, {1.70, 1.62, 1.62}, 3.5}, {128, 128, 1, 0.57, {0.70, 0.70, 0.70}, 2.8}};
 double launch_us(const TileCost& c, int layout, int M, int N, int K, int splits, double per_round, int num_cu) {
     const int wgs = CEIL_DIV(M, c.bm) * CEIL_DIV(N, c.bn) * splits, slots = num_cu * c.per_cu;
-    const int nst = CEIL_DIV(CEIL_DIV(K, PBK), splits), rest = wgs % slots;
+    const int nst = CEIL_DIV(CEIL_DIV(K, RING_K), splits), rest = wgs % slots;
     double stages = (wgs / slots) * c.full[layout];
     if (rest) stages += c.alone + (c.full[layout] - c.alone) * rest / slots;
     const double bytes = ((double)M * K + (double)N * K + (double)M * N * (layout == 2 ? 2 : 1)) * sizeof(floatX);
@@ -338,9 +397,10 @@ constexpr double STAY = 0.96;            // what a ring launch has to come down 
 GemmPlan plan_gemm(int layout, int M, int N, int K, int max_splits, bool small_tiles, double persistent_us, int num_cu) {
     GemmPlan best;
     best.kernel = PERSISTENT_BIG;
-    best.k_per_split = CEIL_DIV(K, PBK) * PBK;
+    best.k_per_split = CEIL_DIV(K, RING_K) * RING_K;
     const size_t big_tiles = (size_t)CEIL_DIV(M, 256) * CEIL_DIV(N, 256);
     if (layout == 2) best.us = persistent_us;
+    else if (sizeof(floatX) == 4) best.us = std::numeric_limits<double>::infinity();      // no persistent kernel
     else {
         if (big_tiles >= 4 * (size_t)num_cu) return best;         // the last round's share is small whatever it is
         best.us = launch_us(PERSISTENT_COST[0], layout, M, N, K, 1, 0.8, num_cu);
@@ -349,18 +409,17 @@ GemmPlan plan_gemm(int layout, int M, int N, int K, int max_splits, bool small_t
             if (us < best.us) { best.us = us; best.kernel = PERSISTENT_SMALL; }
         }
     }
-    const double stay = best.us * STAY;
-    const int stages = CEIL_DIV(K, PBK);
-    double least = stay;
+    const int stages = CEIL_DIV(K, RING_K);
+    double least = best.us * STAY;
     for (int c = 0; c < RING_CFGS; c++) {
         const size_t tiles = (size_t)CEIL_DIV(M, RING_COST[c].bm) * CEIL_DIV(N, RING_COST[c].bn);
-        if (tiles > (size_t)num_cu * 64) continue;
+        if (tiles > (size_t)num_cu * 4096) continue;                // (a grid of 32 bits)
         for (int s = 1; s <= max_splits && s * MIN_STAGES <= std::max(stages, MIN_STAGES); s++) {
             if (s > 1 && (tiles * s > (size_t)num_cu * 4 || CEIL_DIV(stages, CEIL_DIV(stages, s)) != s)) continue;
             const double us = launch_us(RING_COST[c], layout, M, N, K, s, 2.2, num_cu) + (s > 1 ? reduce_us(M, N, s) : 0.0);
             if (us < least) {
                 least = us;
-                best.kernel = c; best.splits = s; best.us = us; best.k_per_split = CEIL_DIV(stages, s) * PBK;
+                best.kernel = c; best.splits = s; best.us = us; best.k_per_split = CEIL_DIV(stages, s) * RING_K;
             }
         }
     }
@@ -379,4 +438,3 @@ void launch_ring(const GemmPlan& plan, GemmArgs g, bool a_t, bool b_t, int epi, 
     else launch_layout<false, false>(plan.kernel, g, epi, rowvec, st);
 }
 }  // namespace gemmk
-#endif

@@ -3,7 +3,6 @@
 #pragma once
 #include "gemm_pipelined.hpp"
 
-#if !defined(LLMK_FP32)
 namespace gemmk {
 
 enum { PERSISTENT_BIG = -1, PERSISTENT_SMALL = -2 };     // 256 x 256 and 128 x 128 tiles of gemm_pipelined.hpp
@@ -13,7 +12,8 @@ struct GemmPlan {
     int k_per_split = 0;
     double us = 1e30;                    // estimated time of the launch and of the pass over its partial products
 };
-// What C[M][N] over K takes. layout: 0 forward, 1 dinp (K multiples of 64), 2 dweight (any K; persistent_us is then the
+constexpr int RING_K = 128 / (int)sizeof(floatX);       // K of a stage: 128 bytes of a row
+// What C[M][N] over K takes. layout: 0 forward, 1 dinp (K multiples of RING_K), 2 dweight (any K; persistent_us is then the
 // estimate of the other way, persistent_tn_us, or infinity where there is none). max_splits: most pieces of K; small_tiles: the
 // 128 x 128 persistent kernel has the epilogue. Arithmetic on the shape alone.
 GemmPlan plan_gemm(int layout, int M, int N, int K, int max_splits, bool small_tiles, double persistent_us, int num_cu);
@@ -23,4 +23,3 @@ double persistent_tn_us(int M, int N, int K, int splits, bool big, int num_cu);
 void launch_ring(const GemmPlan& plan, GemmArgs g, bool a_t, bool b_t, int epi, floatX* rowvec, hipStream_t st);
 
 }  // namespace gemmk
-#endif

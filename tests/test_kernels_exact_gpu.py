@@ -229,24 +229,34 @@ FEW_TILES = [(1, 64, 72), (63, 128, 64), (200, 768, 2304), (333, 384, 1536), (65
              (2331, 384, 1152), (2331, 1536, 384), (3000, 1536, 4608), (4096, 2048, 2048), (4160, 768, 768), (777, 3072, 1024)]
 
 
+@pytest.mark.parametrize("precision", ["bf16", "fp32"])
 @pytest.mark.parametrize("M,C,OC", FEW_TILES)
-def test_projections_of_few_tiles_are_the_integer_products(M, C, OC):
+def test_projections_of_few_tiles_are_the_integer_products(M, C, OC, precision):
     """Forward with each epilogue, dinp with and without GELU backward, dweight and dbias, at sizes that leave part of the chip
-    idle: every product exact, every fused epilogue the same bits as the pass of its own that it stands for."""
+    idle: every product exact, every fused epilogue the same bits as the pass of its own that it stands for (GELU in fp32, where nothing rounds between the
+    product and the function's own operations, to their rounding: a few units of 2^-24)."""
     import torch
-    L = G.lib("bf16")
+    L = G.lib(precision)
+    dt = G.torch_dtype(precision)
+    ints = lambda *a, **k: globals()["ints"](*a, **k).to(dt)
+
+    def same(a, b):
+        return torch.equal(a, b) if precision == "bf16" else torch.allclose(a, b, rtol=1e-6, atol=1e-6)
+
+    def assert_same_bits(got, want, what):
+        assert torch.equal(got, want.to(dt)), what
     x, w, b = ints((M, C), 21, -2, 2), ints((OC, C), 22), ints((OC,), 23, -8, 8)
     lin = exact_nt(x, w) + b.float()
-    out = torch.full((M, OC), 7.0, dtype=torch.bfloat16, device="cuda")
+    out = torch.full((M, OC), 7.0, dtype=dt, device="cuda")
     L.llmk_matmul_forward(G.ptr(out), G.ptr(x), G.ptr(w), G.ptr(b), 1, M, C, OC, None, None, 1)
     G.sync()
     assert_same_bits(out, lin, "x.w^T + b")
-    res = (torch.randn((M, OC), device="cuda") * 3.0).to(torch.bfloat16)
+    res = (torch.randn((M, OC), device="cuda") * 3.0).to(dt)
     L.llmk_matmul_forward_residual(G.ptr(out), G.ptr(x), G.ptr(w), G.ptr(b), G.ptr(res), 1, M, C, OC, None)
     G.sync()
-    assert_same_bits(out, lin.to(torch.bfloat16).float() + res.float(), "x.w^T + b + residual")
+    assert_same_bits(out, lin.to(dt).float() + res.float(), "x.w^T + b + residual")
     ws = ints((OC, C), 22, scale=1.0 / 32)
-    pre_want = (exact_nt(x, ws) + b.float()).to(torch.bfloat16)
+    pre_want = (exact_nt(x, ws) + b.float()).to(dt)
     act_want, grad_want = torch.empty_like(out), torch.ones_like(out)
     L.llmk_gelu_forward(G.ptr(act_want), G.ptr(pre_want), M * OC, None)
     L.llmk_gelu_backward_inplace(G.ptr(grad_want), G.ptr(pre_want), M * OC, None)
@@ -254,7 +264,7 @@ def test_projections_of_few_tiles_are_the_integer_products(M, C, OC):
         pre = torch.zeros_like(out)
         L.llmk_matmul_forward(G.ptr(out), G.ptr(x), G.ptr(ws), G.ptr(b), 1, M, C, OC, None, G.ptr(pre), fusion)
         G.sync()
-        assert torch.equal(pre, kept) and torch.equal(out, act_want), fusion
+        assert same(pre, kept) and same(out, act_want), fusion
     g = ints((M, OC), 24, -2, 2)
     dw0, db0 = ints((OC, C), 25, -50, 50), ints((OC,), 26, -50, 50)
     scratch = torch.empty(max(1, L.llmk_matmul_backward_bias_scratch_floats(OC)), dtype=torch.float32, device="cuda")
@@ -262,14 +272,14 @@ def test_projections_of_few_tiles_are_the_integer_products(M, C, OC):
     dw_want, db_want = dw0.float() + exact_tn(g, x), db0.float() + g.float().sum(0)
     kept = ints((M, C), 27, -24, 24, scale=1.0 / 8)
     for fusion in (None, 0, 2, 3):
-        dx, dw, db = torch.full((M, C), 7.0, dtype=torch.bfloat16, device="cuda"), dw0.clone(), db0.clone()
+        dx, dw, db = torch.full((M, C), 7.0, dtype=dt, device="cuda"), dw0.clone(), db0.clone()
         L.llmk_matmul_backward(G.ptr(dx), G.ptr(dw), G.ptr(db) if fusion != 2 else None, G.ptr(g), G.ptr(x), G.ptr(w), G.ptr(scratch),
                                1, M, C, OC, None, None if fusion is None else G.ptr(kept), 1 if fusion is None else fusion)
-        want = dx_want.to(torch.bfloat16)
-        if fusion == 3: want = (want.float() * kept.float()).to(torch.bfloat16)
+        want = dx_want.to(dt, copy=True)
+        if fusion == 3: want = (want.float() * kept.float()).to(dt)
         elif fusion is not None: L.llmk_gelu_backward_inplace(G.ptr(want), G.ptr(kept), M * C, None)
         G.sync()
-        assert torch.equal(dx, want), ("dinp", fusion)
+        assert same(dx, want), ("dinp", fusion)
         assert_same_bits(dw, dw_want, "dweight")
         assert_same_bits(db, db_want if fusion != 2 else db0.float(), "dbias")
     G.check_no_error(L)
