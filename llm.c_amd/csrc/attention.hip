@@ -1494,9 +1494,9 @@ void attention_backward_impl(void* dqkvr, const void* dout, const void* qkvr, co
 namespace llmk {
 void attention_static_scratch_init() { (void)static_scratch_setup(); }
 
-// One sequence, queries t0 .. T - 1 (t0 a multiple of 32, T - t0 at most 32) against keys 0 .. T - 1, with the bits that a
-// sampled token has always depended on. Heads of 64: the matrix-core kernel runs the query tile that holds the rows, one
-// workgroup per head; the rows of that tile before t0 come out again as they were. Others: one wave per row.
+// One sequence, query T - 1 against keys 0 .. T - 1, with the bits that a sampled token has always depended on; t0: T - 1 rounded
+// down to a multiple of 32. Heads of 64, and fp32: the matrix-core kernels run the query tile that holds the row, one workgroup
+// per head; the rows of that tile before it come out again as they were. Others: one wave per head.
 void decode_attention(void* out, const void* qkv, int t0, int T, int NH, int C, hipStream_t st) {
     if (failed()) return;
     const int hs = C / NH;
@@ -1506,6 +1506,7 @@ void decode_attention(void* out, const void* qkv, int t0, int T, int NH, int C, 
         LAUNCH_CHECK();
         return;
     }
+    t0 = T - 1;
 #endif
     launch_forward_rows((floatX*)out, nullptr, (const floatX*)qkv, 1, T, NH, hs, t0, st);
     LAUNCH_CHECK();

@@ -94,7 +94,7 @@ struct LLMK_GPT2 {
     int gelu_fusion = 0, recompute = 1;
     int* workload_indices = nullptr;
     int* bucket_info = nullptr;
-    char* decode_host = nullptr;               // pinned: the 32 tokens and the logits row of a generation step
+    char* decode_host = nullptr;               // pinned: the token and the logits row of a generation step
     hipStream_t stream = nullptr;
 };
 
@@ -525,57 +525,42 @@ float gpt2_validate(LLMK_GPT2* m, const int* inputs, const int* targets, size_t 
 }
 
 namespace {
-constexpr int DECODE_ROWS = 32;                // rows of one generation step: the row block of the matrix kernels
+constexpr int DECODE_ROWS = 32;                // rows that the attention kernels take at a time
 
-// The forward pass of positions r0 .. r0 + n - 1 of one sequence (r0 a multiple of DECODE_ROWS, n at most that) whose earlier
-// positions have been through here: their K and V lie in the qkvr tensor, layer by layer, seq_len rows each. Everything else
-// is needed for these rows only and goes through the first rows of the activation tensors. A row's result depends on its own
-// inputs and the K and V before it, and every kernel adds up in the order of the full forward pass: the same bits. Leaves the
-// logits of the rows at output + r0 rows. tokens: device-visible, the n tokens.
-void decode_block(LLMK_GPT2* m, const int* tokens, int r0, int n) {
+// The forward pass of position r of one sequence whose earlier positions have been through here: their K and V lie in the qkvr
+// tensor, layer by layer, seq_len rows each. Everything else is needed for this row only and goes through the first rows of the
+// activation tensors. A row's result depends on its own inputs and the K and V before it, and every kernel adds up in the
+// order of the full forward pass: the same bits. Leaves the logits at row r of output. token: device-visible.
+void decode_row(LLMK_GPT2* m, const int* token, int r) {
     const size_t Vp = m->config.padded_vocab_size, L = m->config.num_layers, C = m->config.channels, X = m->X, T = m->seq_len;
-    const int NH = m->config.num_heads;
+    const int NH = m->config.num_heads, iC = (int)C;
     hipStream_t st = m->stream;
     const ParameterTensors p = m->params;
     const ActivationTensors a = m->acts;
-    const xptr ln = a.lnf, atty = off(a.atty, (size_t)r0 * C, X), scratch = a.output;
-    llmk_encoder_forward(a.encoded, tokens, p.wte, off(p.wpe, (size_t)r0 * C, X), 1, n, (int)C, st);
-    llmk_layernorm_forward(ln, nullptr, nullptr, a.encoded, p.ln1w, p.ln1b, 1, n, (int)C, st);
+    const xptr ln = a.lnf, atty = off(a.atty, (size_t)r * C, X);
+    llmk_encoder_forward(a.encoded, token, p.wte, off(p.wpe, (size_t)r * C, X), 1, 1, iC, st);
     xptr residual = a.encoded;
     for (size_t l = 0; l < L; l++) {
         const xptr qkv = off(a.qkvr, l * T * 3 * C, X);
-        llmk::decode_matmul(off(qkv, (size_t)r0 * 3 * C, X), ln, off(p.qkvw, l * 3 * C * C, X), off(p.qkvb, l * 3 * C, X), nullptr, nullptr,
-                            n, (int)C, (int)(3 * C), st);
-        llmk::decode_attention(a.atty, qkv, r0, r0 + n, NH, (int)C, st);
-        const xptr n_w = l + 1 != L ? off(p.ln1w, (l + 1) * C, X) : p.lnfw, n_b = l + 1 != L ? off(p.ln1b, (l + 1) * C, X) : p.lnfb;
-        const xptr ln2w = off(p.ln2w, l * C, X), ln2b = off(p.ln2b, l * C, X);
-        const xptr attprojw = off(p.attprojw, l * C * C, X), attprojb = off(p.attprojb, l * C, X);
-        const xptr fcw = off(p.fcw, l * 4 * C * C, X), fcb = off(p.fcb, l * 4 * C, X);
-        const xptr fcprojw = off(p.fcprojw, l * C * 4 * C, X), fcprojb = off(p.fcprojb, l * C, X);
-        if (X == 2) {                              // as in forward_impl: the adds are the projections' epilogues
-            llmk::decode_matmul(a.residual2, atty, attprojw, attprojb, nullptr, residual, n, (int)C, (int)C, st);
-            llmk_layernorm_forward(ln, nullptr, nullptr, a.residual2, ln2w, ln2b, 1, n, (int)C, st);
-            llmk::decode_matmul(a.fch_gelu, ln, fcw, fcb, a.fch, nullptr, n, (int)C, (int)(4 * C), st);
-            llmk::decode_matmul(a.residual3, a.fch_gelu, fcprojw, fcprojb, nullptr, a.residual2, n, (int)(4 * C), (int)C, st);
-            llmk_layernorm_forward(ln, nullptr, nullptr, a.residual3, n_w, n_b, 1, n, (int)C, st);
-        } else {
-            llmk::decode_matmul(scratch, atty, attprojw, attprojb, nullptr, nullptr, n, (int)C, (int)C, st);
-            llmk_fused_residual_forward5(a.residual2, ln, nullptr, nullptr, residual, scratch, ln2w, ln2b, n, (int)C, st);
-            llmk::decode_matmul(a.fch_gelu, ln, fcw, fcb, a.fch, nullptr, n, (int)C, (int)(4 * C), st);
-            llmk::decode_matmul(scratch, a.fch_gelu, fcprojw, fcprojb, nullptr, nullptr, n, (int)(4 * C), (int)C, st);
-            llmk_fused_residual_forward5(a.residual3, ln, nullptr, nullptr, a.residual2, scratch, n_w, n_b, n, (int)C, st);
-        }
+        llmk::decode_matmul(off(qkv, (size_t)r * 3 * C, X), ln, residual, off(p.ln1w, l * C, X), off(p.ln1b, l * C, X), off(p.qkvw, l * 3 * C * C, X),
+                            off(p.qkvb, l * 3 * C, X), nullptr, nullptr, iC, 3 * iC, st);
+        llmk::decode_attention(a.atty, qkv, r / DECODE_ROWS * DECODE_ROWS, r + 1, NH, iC, st);
+        llmk::decode_matmul(a.residual2, nullptr, atty, nullptr, nullptr, off(p.attprojw, l * C * C, X), off(p.attprojb, l * C, X), nullptr, residual,
+                            iC, iC, st);
+        llmk::decode_matmul(a.fch_gelu, ln, a.residual2, off(p.ln2w, l * C, X), off(p.ln2b, l * C, X), off(p.fcw, l * 4 * C * C, X),
+                            off(p.fcb, l * 4 * C, X), a.fch, nullptr, iC, 4 * iC, st);
+        llmk::decode_matmul(a.residual3, nullptr, a.fch_gelu, nullptr, nullptr, off(p.fcprojw, l * C * 4 * C, X), off(p.fcprojb, l * C, X), nullptr,
+                            a.residual2, 4 * iC, iC, st);
         residual = a.residual3;
     }
-    llmk::decode_matmul(off(a.output, (size_t)r0 * Vp, X), ln, p.wte, nullptr, nullptr, nullptr, n, (int)C, (int)Vp, st);
+    llmk::decode_matmul(off(a.output, (size_t)r * Vp, X), ln, residual, p.lnfw, p.lnfb, p.wte, nullptr, nullptr, nullptr, iC, (int)Vp, st);
 }
 }  // namespace
 
 // The generation loop of the reference's trainer (train_gpt2.cu:1751-1796), without the printing: every position of
 // gen_tokens starts as eot_token, then positions 1..genT-1 are drawn one at a time from the model's distribution after
 // the tokens before them. The reference runs the whole sequence, rounded up to a multiple of 256, for every draw; here a draw
-// runs the block of 32 rows that its position lies in, on the K and V of the rows before (decode_block). The logits of the last
-// real position move to the host and are sampled there with llmc/sampler.h's generator, whose state the caller owns (the
+// runs the one row that is new, on the K and V of the rows before (decode_row). Its logits move to the host and are sampled there with llmc/sampler.h's generator, whose state the caller owns (the
 // reference starts it at 1337 for every generation).
 void gpt2_generate(LLMK_GPT2* m, int* gen_tokens, int genT, int eot_token, unsigned long long* sample_rng_state) {
     const int B = m->batch_size, T = m->seq_len, V = m->config.vocab_size;
@@ -585,19 +570,16 @@ void gpt2_generate(LLMK_GPT2* m, int* gen_tokens, int genT, int eot_token, unsig
     for (int i = 0; i < B * T; i++) gen_tokens[i] = eot_token;
     if (genT > 1) token_check(&eot_token, 1, V);
     const size_t row_bytes = (size_t)V * m->X;
-    if (!m->decode_host) hipCheck(hipHostMalloc((void**)&m->decode_host, DECODE_ROWS * sizeof(int) + row_bytes));
-    int* tokens = (int*)m->decode_host;
-    char* raw = m->decode_host + DECODE_ROWS * sizeof(int);
-    std::vector<float> cpu_logits(V);
+    if (!m->decode_host) hipCheck(hipHostMalloc((void**)&m->decode_host, 64 + row_bytes));
+    int* token = (int*)m->decode_host;
+    char* raw = m->decode_host + 64;
+    llmk::SoftmaxSampler sampler(V, m->X == 2);
     for (int t = 1; t < genT; t++) {
-        const int r0 = (t - 1) / DECODE_ROWS * DECODE_ROWS, n = std::min(DECODE_ROWS, T - r0);
-        memcpy(tokens, gen_tokens + r0, n * sizeof(int));      // the stream is idle here: the step before has been waited for
-        decode_block(m, tokens, r0, n);
+        *token = gen_tokens[t - 1];                            // the stream is idle here: the step before has been waited for
+        decode_row(m, token, t - 1);
         hipCheck(hipMemcpyAsync(raw, off(m->acts.output, (size_t)(t - 1) * Vp, m->X), row_bytes, hipMemcpyDeviceToHost, m->stream));
         hipCheck(hipStreamSynchronize(m->stream));
-        from_storage(cpu_logits.data(), raw, V, m->X);
-        const float coin = llmk::random_f32(sample_rng_state);
-        gen_tokens[t] = llmk::sample_softmax(cpu_logits.data(), V, coin);
+        gen_tokens[t] = sampler.draw(raw, llmk::random_f32(sample_rng_state));
     }
 }
 
