@@ -20,9 +20,12 @@ __device__ const u32x4 g_zero_chunk = {0, 0, 0, 0};
 // What bounds it: a lone workgroup draws 25 bytes a clock from L2 whatever its tile and however deep the ring, so few tiles want
 // to be many small ones (the fourfold traffic of 64 x 64 is spread over more CUs); a full chip wants 256 x 128, whose 96 KiB of
 // stages in flight leave no epilogue to overlap with, which is why the persistent kernel keeps launches of many tiles.
+// Wave tiles are 64 x 32 or 32 x 64 (32 x 32 in the two smallest): twice the waves of 64 x 64 ones read half as much again from LDS
+// and hide its latency and the loads' issue from each other: 3885 x 1024 over 4096 40.8 -> 37.0 us, dweight 2048 x 2048 over 4096
+// 48.6 -> 41.8, 3000 x 1536 over 4608 60 -> 53.
 // Measured, weights from HBM, us, the persistent kernel's better tile against this: 256 x 768 over K = 3072 29.6 / 15.0 (one
-// piece), 9.9 (four, with the pass over the partials), over K = 50304 613 / 42; 4096 x 2048 over 8192 156 / 123; 3000 x 1536 over
-// 6144 120 / 82; dweight 3072 x 768 over 256 rows 19.7 / 7.1, 4608 x 1536 over 3000 rows (no persistent kernel) 83 / 52.
+// piece), 9.9 (four, with the pass over the partials), over K = 50304 613 / 42; 4096 x 2048 over 8192 156 / 124; 3000 x 1536 over
+// 6144 120 / 80; dweight 3072 x 768 over 256 rows 19.7 / 7.1, 4608 x 1536 over 3000 rows (no persistent kernel) 83 / 52.
 // The fp32 library has the same kernel with the fp32 matrix instruction, 16 of which make a stage of 32: the matrix cores bound
 // it (2048 x 50304 over 768: 119 TFLOP/s of 157) as soon as every CU has a tile, so what counts is tiles small enough for that.
 constexpr int CE = 16 / (int)sizeof(floatX);     // elements of a 16-byte chunk
@@ -347,10 +350,10 @@ void launch_cfg(const GemmArgs& g, int epi, floatX* rowvec, hipStream_t st) {
 template <bool A_T, bool B_T>
 void launch_layout(int cfg, const GemmArgs& g, int epi, floatX* rowvec, hipStream_t st) {
     switch (cfg) {
-        case 0: launch_cfg<256, 128, 4, 2, 3, A_T, B_T>(g, epi, rowvec, st); break;
-        case 1: launch_cfg<128, 128, 2, 2, 2, A_T, B_T>(g, epi, rowvec, st); break;
-        case 2: launch_cfg<128, 128, 2, 2, 4, A_T, B_T>(g, epi, rowvec, st); break;
-        case 3: launch_cfg<128, 64, 2, 2, 3, A_T, B_T>(g, epi, rowvec, st); break;
+        case 0: launch_cfg<256, 128, 4, 4, 3, A_T, B_T>(g, epi, rowvec, st); break;
+        case 1: launch_cfg<128, 128, 2, 4, 2, A_T, B_T>(g, epi, rowvec, st); break;
+        case 2: launch_cfg<128, 128, 4, 2, 4, A_T, B_T>(g, epi, rowvec, st); break;
+        case 3: launch_cfg<128, 64, 4, 2, 3, A_T, B_T>(g, epi, rowvec, st); break;
         case 4: launch_cfg<64, 64, 2, 2, 3, A_T, B_T>(g, epi, rowvec, st); break;
         default: LLMK_REQUIRE(false, "launch_ring: no configuration %d", cfg);
     }
@@ -372,10 +375,10 @@ constexpr TileCost RING_COST[RING_CFGS] = {
 };
 #else
 constexpr TileCost RING_COST[RING_CFGS] = {
-    {256, 128, 1, 0.75, {0.97, 0.95, 1.12}, 5.0},
-    {128, 128, 2, 0.57, {0.96, 1.09, 1.10}, 4.5},
-    {128, 128, 1, 0.57, {0.65, 0.61, 0.72}, 4.5},
-    {128, 64, 2, 0.39, {0.62, 0.62, 0.72}, 3.6},
+    {256, 128, 1, 0.72, {0.94, 0.92, 1.05}, 5.0},
+    {128, 128, 2, 0.46, {0.95, 1.02, 1.05}, 4.2},
+    {128, 128, 1, 0.45, {0.57, 0.53, 0.60}, 4.2},
+    {128, 64, 2, 0.32, {0.61, 0.61, 0.70}, 3.4},
     {64, 64, 3, 0.29, {0.58, 0.58, 0.64}, 2.8},
 };
 #endif
