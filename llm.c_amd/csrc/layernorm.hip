@@ -10,6 +10,7 @@
 // and — in the fused kernel — statistics of the residual AFTER rounding it to the storage
 // type (llmc/layernorm.cuh:178-184).
 #include "common.hpp"
+#include "layernorm.hpp"
 #include "../../include/llmk.h"
 
 namespace {
@@ -210,7 +211,7 @@ residual_kernel(floatX* __restrict__ out, const floatX* __restrict__ a, const fl
 
 // ---- backward ------------------------------------------------------------------------------
 // Each wave walks rows; per-lane fp32 accumulators hold dweight/dbias of the lane's columns.
-// At the end the 4 waves of a workgroup are added in wave order through LDS and the workgroup's
+// At the end the waves of a workgroup are added in wave order through LDS and the workgroup's
 // partial goes to scratch[block][2][C]; a second kernel adds the partials in block order, so
 // the result does not depend on scheduling (no atomics).
 // One workgroup per CU, as many waves as the accumulators leave room for: 12 (three per SIMD) up to NV = 2, where the
@@ -225,7 +226,7 @@ ln_backward_kernel(floatX* __restrict__ dinp, float* __restrict__ partial, const
                    const floatX* __restrict__ inp, const floatX* __restrict__ weight,
                    const float* __restrict__ mean, const float* __restrict__ rstd, int N, int C) {
     constexpr int LNB_WAVES = lnb_waves(NV);
-    extern __shared__ float lds[];   // [LNB_WAVES-1][2][C]
+    extern __shared__ float lds[];   // [LNB_WAVES][2][C]
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
     const int wave = blockIdx.x * LNB_WAVES + wid;
@@ -331,37 +332,25 @@ ln_backward_kernel(floatX* __restrict__ dinp, float* __restrict__ partial, const
         }
     }
 
-    // workgroup reduction in fixed wave order
-    if (wid > 0) {
-        float* dst = lds + (size_t)(wid - 1) * 2 * C;
+    // workgroup reduction in fixed wave order, the columns dealt to all lanes (before, one wave added up the others' sums, eight
+    // columns to a lane). With this and the one launch for all LayerNorms' sums below, a 124M step at 4 x 64 2996 -> 2851 us,
+    // at 4 x 1024 7835 -> 7653, 350M at 2 x 16 x 1024 85.2 -> 84.1 ms (that one with another choice of GEMM as well).
+    float* dst = lds + (size_t)wid * 2 * C;
 #pragma unroll
-        for (int i = 0; i < NV; i++) {
-            int v = lane + i * 64;
-            if (v < nvec) {
+    for (int i = 0; i < NV; i++) {
+        int v = lane + i * 64;
+        if (v < nvec) {
 #pragma unroll
-                for (int k = 0; k < VN; k++) { dst[v * VN + k] = dw[i][k]; dst[C + v * VN + k] = db[i][k]; }
-            }
+            for (int k = 0; k < VN; k++) { dst[v * VN + k] = dw[i][k]; dst[C + v * VN + k] = db[i][k]; }
         }
     }
     __syncthreads();
-    if (wid == 0) {
-        float* out = partial + (size_t)blockIdx.x * 2 * C;
+    float* out = partial + (size_t)blockIdx.x * 2 * C;
+    for (int c = threadIdx.x; c < 2 * C; c += LNB_WAVES * 64) {
+        float s = lds[c];
 #pragma unroll
-        for (int i = 0; i < NV; i++) {
-            int v = lane + i * 64;
-            if (v < nvec) {
-#pragma unroll
-                for (int k = 0; k < VN; k++) {
-                    float sw = dw[i][k], sb = db[i][k];
-                    for (int o = 0; o < LNB_WAVES - 1; o++) {
-                        sw += lds[(size_t)o * 2 * C + v * VN + k];
-                        sb += lds[(size_t)o * 2 * C + C + v * VN + k];
-                    }
-                    out[v * VN + k] = sw;
-                    out[C + v * VN + k] = sb;
-                }
-            }
-        }
+        for (int o = 1; o < LNB_WAVES; o++) s += lds[(size_t)o * 2 * C + c];
+        out[c] = s;
     }
 }
 
@@ -421,13 +410,16 @@ ln_backward_wide_kernel(floatX* __restrict__ dinp, float* __restrict__ partial, 
 // groups each add every 32nd partial in ascending order, then the 32 sub-sums are added in group order:
 // a fixed summation tree, so the result is reproducible, with 32x the memory parallelism of one thread
 // per column.
+//
+// One launch can do this for several LayerNorms (blockIdx.y), as the driver has it at the end of a backward pass: for one it is all
+// start and end, and there are two to a layer. The 25 of the 124M model together: 5.0 us at 256 rows, 17 at 4096.
 constexpr int LNR_COLS = 32, LNR_GROUPS = 32;
 __global__ void __launch_bounds__(LNR_COLS * LNR_GROUPS)
-ln_backward_reduce_kernel(floatX* __restrict__ dweight, floatX* __restrict__ dbias, const float* __restrict__ partial,
-                          int nblocks, int C) {
+ln_backward_reduce_kernel(llmk::LnGrads grads, const float* __restrict__ partial, int nblocks, int C) {
     __shared__ float sub[LNR_GROUPS][LNR_COLS];
     const int cl = threadIdx.x % LNR_COLS, grp = threadIdx.x / LNR_COLS;
-    const int c = blockIdx.x * LNR_COLS + cl;
+    const int c = blockIdx.x * LNR_COLS + cl, n = blockIdx.y;
+    partial += (size_t)n * nblocks * 2 * C;
     float s = 0.f;
     if (c < 2 * C)
         for (int b = grp; b < nblocks; b += LNR_GROUPS) s += partial[(size_t)b * 2 * C + c];
@@ -437,14 +429,70 @@ ln_backward_reduce_kernel(floatX* __restrict__ dweight, floatX* __restrict__ dbi
         float t = 0.f;
 #pragma unroll
         for (int g2 = 0; g2 < LNR_GROUPS; g2++) t += sub[g2][cl];
-        floatX* dst = c < C ? dweight + c : dbias + (c - C);
+        const int kind = min(n / grads.layers, 2);
+        const size_t layer = (size_t)(n - kind * grads.layers) * C;
+        floatX* dst = c < C ? (floatX*)grads.dweight[kind] + layer + c : (floatX*)grads.dbias[kind] + layer + (c - C);
         *dst = from_f32<floatX>(to_f32(*dst) + t);
     }
 }
 
 int ln_backward_blocks() { return llmk::device_info().num_cu; }
+constexpr int LNB_MAX_VECS = 8;               // vectors per lane of the register-resident kernel
 
 }  // namespace
+
+namespace llmk {
+int layernorm_backward_partials(int N, int C) {
+    const int nv = CEIL_DIV(C / VN, 64);
+    return min(ln_backward_blocks(), nv > LNB_MAX_VECS ? N : CEIL_DIV(N, lnb_waves(nv)));
+}
+
+void layernorm_backward_rows(void* dinp, float* partial, const void* dout, const void* inp, const void* weight, const float* mean,
+                             const float* rstd, int N, int C, hipStream_t st) {
+    if (failed()) return;
+    LLMK_REQUIRE(C > 0 && C % VN == 0, "layernorm_backward: C=%d must be a multiple of %d", C, VN);
+    if (N == 0) return;
+    const int nv = CEIL_DIV(C / VN, 64), blocks = layernorm_backward_partials(N, C);
+    if (nv > LNB_MAX_VECS) {                                  // wider than the register-resident kernel takes
+        const size_t smem = (2 * (size_t)C + 32) * sizeof(float);
+        LLMK_REQUIRE(smem <= 160 * 1024, "layernorm_backward: C=%d too large (max %d)", C, (160 * 1024 / 4 - 32) / 2);
+        ProfScope prof("layernorm_backward", 0, 4.0 * N * C * sizeof(floatX) + 2.0 * N * sizeof(float), st);
+        static bool attr_set = false;
+        if (!attr_set) {
+            HIP_CHECK(hipFuncSetAttribute((const void*)ln_backward_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            attr_set = true;
+        }
+        ln_backward_wide_kernel<<<blocks, 256, smem, st>>>((floatX*)dinp, partial, (const floatX*)dout, (const floatX*)inp,
+                                                           (const floatX*)weight, mean, rstd, N, C);
+        LAUNCH_CHECK();
+        return;
+    }
+    const size_t smem = (size_t)lnb_waves(nv) * 2 * C * sizeof(float);
+    ProfScope prof("layernorm_backward", 0, 4.0 * N * C * sizeof(floatX) + 2.0 * N * sizeof(float), st);
+#define LNB_CASE(K)                                                                                          \
+    case K: {                                                                                                \
+        static bool attr_set = false;                                                                        \
+        if (!attr_set) {                                                                                     \
+            HIP_CHECK(hipFuncSetAttribute((const void*)ln_backward_kernel<K>,                                \
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));          \
+            attr_set = true;                                                                                 \
+        }                                                                                                    \
+        ln_backward_kernel<K><<<blocks, lnb_waves(K) * 64, smem, st>>>((floatX*)dinp, partial, (const floatX*)dout, \
+                                                              (const floatX*)inp, (const floatX*)weight,    \
+                                                              mean, rstd, N, C);                             \
+        break; }
+    switch (nv) { LNB_CASE(1) LNB_CASE(2) LNB_CASE(3) LNB_CASE(4) LNB_CASE(5) LNB_CASE(6) LNB_CASE(7) LNB_CASE(8) }
+#undef LNB_CASE
+    LAUNCH_CHECK();
+}
+
+void layernorm_backward_reduce(const LnGrads& grads, int count, const float* partial, int blocks, int C, hipStream_t st) {
+    if (failed() || count == 0 || blocks == 0) return;
+    ProfScope prof("layernorm_backward_reduce", 0, (double)count * blocks * 2 * C * sizeof(float), st);
+    ln_backward_reduce_kernel<<<dim3(CEIL_DIV(2 * C, LNR_COLS), count), LNR_COLS * LNR_GROUPS, 0, st>>>(grads, partial, blocks, C);
+    LAUNCH_CHECK();
+}
+}  // namespace llmk
 
 extern "C" {
 
@@ -483,56 +531,12 @@ size_t llmk_layernorm_backward_scratch_floats(int C) { return (size_t)ln_backwar
 void llmk_layernorm_backward(void* dinp, void* dweight, void* dbias, float* scratch, const void* dout,
                              const void* inp, const void* weight, const float* mean, const float* rstd, int B,
                              int T, int C, void* stream) {
-    if (llmk::failed()) return;
-    LLMK_REQUIRE(C > 0 && C % VN == 0, "layernorm_backward: C=%d must be a multiple of %d", C, VN);
-    const int nv = CEIL_DIV(C / VN, 64);
     const int N = B * T;
-    if (N == 0) return;
     hipStream_t st = (hipStream_t)stream;
-    if (nv > 8) {                                             // wider than the register-resident kernel takes
-        const size_t smem = (2 * (size_t)C + 32) * sizeof(float);
-        LLMK_REQUIRE(smem <= 160 * 1024, "layernorm_backward: C=%d too large (max %d)", C, (160 * 1024 / 4 - 32) / 2);
-        const int blocks = min(ln_backward_blocks(), N);
-        {
-            llmk::ProfScope prof("layernorm_backward", 0, 4.0 * N * C * sizeof(floatX) + 2.0 * N * sizeof(float), st);
-            static bool attr_set = false;
-            if (!attr_set) {
-                HIP_CHECK(hipFuncSetAttribute((const void*)ln_backward_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-                attr_set = true;
-            }
-            ln_backward_wide_kernel<<<blocks, 256, smem, st>>>((floatX*)dinp, scratch, (const floatX*)dout, (const floatX*)inp,
-                                                             (const floatX*)weight, mean, rstd, N, C);
-            LAUNCH_CHECK();
-        }
-        llmk::ProfScope prof2("layernorm_backward_reduce", 0, (double)blocks * 2 * C * sizeof(float), st);
-        ln_backward_reduce_kernel<<<CEIL_DIV(2 * C, LNR_COLS), LNR_COLS * LNR_GROUPS, 0, st>>>((floatX*)dweight, (floatX*)dbias, scratch, blocks, C);
-        LAUNCH_CHECK();
-        return;
-    }
-    const int waves = lnb_waves(nv);
-    const int blocks = min(ln_backward_blocks(), CEIL_DIV(N, waves));
-    const size_t smem = (size_t)(waves - 1) * 2 * C * sizeof(float);
-    {
-    llmk::ProfScope prof("layernorm_backward", 0, 4.0 * N * C * sizeof(floatX) + 2.0 * N * sizeof(float), st);
-#define LNB_CASE(K)                                                                                          \
-    case K: {                                                                                                \
-        static bool attr_set = false;                                                                        \
-        if (!attr_set) {                                                                                     \
-            HIP_CHECK(hipFuncSetAttribute((const void*)ln_backward_kernel<K>,                                \
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));          \
-            attr_set = true;                                                                                 \
-        }                                                                                                    \
-        ln_backward_kernel<K><<<blocks, lnb_waves(K) * 64, smem, st>>>((floatX*)dinp, scratch, (const floatX*)dout, \
-                                                              (const floatX*)inp, (const floatX*)weight,    \
-                                                              mean, rstd, N, C);                             \
-        break; }
-    switch (nv) { LNB_CASE(1) LNB_CASE(2) LNB_CASE(3) LNB_CASE(4) LNB_CASE(5) LNB_CASE(6) LNB_CASE(7) LNB_CASE(8) }
-#undef LNB_CASE
-    LAUNCH_CHECK();
-    }
-    llmk::ProfScope prof2("layernorm_backward_reduce", 0, (double)blocks * 2 * C * sizeof(float), st);
-    ln_backward_reduce_kernel<<<CEIL_DIV(2 * C, LNR_COLS), LNR_COLS * LNR_GROUPS, 0, st>>>((floatX*)dweight, (floatX*)dbias, scratch, blocks, C);
-    LAUNCH_CHECK();
+    llmk::layernorm_backward_rows(dinp, scratch, dout, inp, weight, mean, rstd, N, C, st);
+    if (N == 0) return;
+    const llmk::LnGrads grads = {{dweight, nullptr, nullptr}, {dbias, nullptr, nullptr}, 1};
+    llmk::layernorm_backward_reduce(grads, 1, scratch, llmk::layernorm_backward_partials(N, C), C, st);
 }
 
 }  // extern "C"

@@ -25,6 +25,7 @@
 #include "../../include/llmk_gpt2.h"
 #include "../../include/llmk_data.h"
 #include "../csrc/decode.hpp"
+#include "../csrc/layernorm.hpp"
 #include "rand.hpp"
 
 #define hipCheck(expr)                                                                            \
@@ -525,7 +526,7 @@ float gpt2_validate(LLMK_GPT2* m, const int* inputs, const int* targets, size_t 
 }
 
 namespace {
-constexpr int DECODE_ROWS = 32;                // rows that the attention kernels take at a time
+constexpr int DECODE_ROWS = 32;                // rows that the attention kernels take at a time (decode_attention)
 
 // The forward pass of position r of one sequence whose earlier positions have been through here: their K and V lie in the qkvr
 // tensor, layer by layer, seq_len rows each. Everything else is needed for this row only and goes through the first rows of the
@@ -560,8 +561,9 @@ void decode_row(LLMK_GPT2* m, const int* token, int r) {
 // The generation loop of the reference's trainer (train_gpt2.cu:1751-1796), without the printing: every position of
 // gen_tokens starts as eot_token, then positions 1..genT-1 are drawn one at a time from the model's distribution after
 // the tokens before them. The reference runs the whole sequence, rounded up to a multiple of 256, for every draw; here a draw
-// runs the one row that is new, on the K and V of the rows before (decode_row). Its logits move to the host and are sampled there with llmc/sampler.h's generator, whose state the caller owns (the
-// reference starts it at 1337 for every generation).
+// runs the one row that is new, on the K and V of the rows before (decode_row). Its logits move to the host and are sampled
+// there with llmc/sampler.h's generator, whose state the caller owns (the reference starts it at 1337 for every generation).
+// 64 tokens from the 124M model: 97.1 -> 29.4 ms; a token is 62 launches, none shorter than 4 us, and 54 us of sampling.
 void gpt2_generate(LLMK_GPT2* m, int* gen_tokens, int genT, int eot_token, unsigned long long* sample_rng_state) {
     const int B = m->batch_size, T = m->seq_len, V = m->config.vocab_size;
     const size_t Vp = m->config.padded_vocab_size;
@@ -607,10 +609,25 @@ void backward_impl(LLMK_GPT2* m, const int* inputs, const int* targets, int grad
     token_check(targets, B * T, (int)V);
     llmk_fused_classifier(a.output, a.losses, dloss, m->targets, (int)B, (int)T, (int)V, (int)Vp, 1, st);
     float* scratchF = (float*)a.output;
+    // The logits buffer, free from the LM head's backward on, is also where the LayerNorms leave their partial sums of dweight and
+    // dbias, all of them behind the scratch of the other launchers, to be added up by one launch at the end instead of one each.
+    // Where they do not fit (deep models of a small vocabulary) each is added up on its own. The same bits either way.
+    const int N = (int)(B * T), num_ln = 2 * (int)L + 1, ln_blocks = llmk::layernorm_backward_partials(N, (int)C);
+    size_t scratch_floats = 0;
+    for (size_t oc : {C, 3 * C, 4 * C}) scratch_floats = std::max(scratch_floats, llmk_matmul_backward_bias_scratch_floats((int)oc));
+    float* ln_partials = scratchF + ceil_div(scratch_floats, 64) * 64;
+    const size_t ln_floats = (size_t)ln_blocks * 2 * C;
+    const bool ln_together = (char*)(ln_partials + ln_floats * num_ln) <= (char*)a.output + m->acts_specs[18].size * X;
+    const llmk::LnGrads ln_grads = {{g.ln1w, g.ln2w, g.lnfw}, {g.ln1b, g.ln2b, g.lnfb}, (int)L};
+    // n: 0 .. L - 1 the first LayerNorms of the layers, then the second ones, then the last
+    auto layernorm_backward = [&](int n, xptr dweight, xptr dbias, xptr dout, xptr inp, xptr weight, float* mean, float* rstd) {
+        if (ln_together) llmk::layernorm_backward_rows(dresidual, ln_partials + n * ln_floats, dout, inp, weight, mean, rstd, N, (int)C, st);
+        else llmk_layernorm_backward(dresidual, dweight, dbias, scratchF, dout, inp, weight, mean, rstd, (int)B, (int)T, (int)C, st);
+    };
 
     llmk_matmul_backward(a.scratch_bt4c, g.wte, nullptr, a.output, a.lnf, p.wte, nullptr, (int)B, (int)T, (int)C, (int)Vp, st, nullptr, 1);
     xptr residual = off(a.residual3, (L - 1) * B * T * C, X);
-    llmk_layernorm_backward(dresidual, g.lnfw, g.lnfb, scratchF, a.scratch_bt4c, residual, p.lnfw, a.lnf_mean, a.lnf_rstd, (int)B, (int)T, (int)C, st);
+    layernorm_backward(2 * (int)L, g.lnfw, g.lnfb, a.scratch_bt4c, residual, p.lnfw, a.lnf_mean, a.lnf_rstd);
     xptr dl_btc = residual;   // the last residual is dead from here on: generic (B,T,C) scratch
 
     for (int l = (int)L - 1; l >= 0; l--) {
@@ -643,14 +660,15 @@ void backward_impl(LLMK_GPT2* m, const int* inputs, const int* targets, int grad
         llmk_matmul_backward(dl_bt4c, dl_fcprojw, dl_fcprojb, dresidual, l_fch_gelu, l_fcprojw, scratchF, (int)B, (int)T, (int)(4 * C), (int)C, st, l_fch_pre_gelu, gelu_fusion_in_use(m));
         if (R >= 2) llmk_layernorm_forward(l_ln2, l_ln2_mean, l_ln2_rstd, l_residual2, l_ln2w, l_ln2b, (int)B, (int)T, (int)C, st);
         llmk_matmul_backward(dl_btc, dl_fcw, dl_fcb, dl_bt4c, l_ln2, l_fcw, scratchF, (int)B, (int)T, (int)C, (int)(4 * C), st, nullptr, 1);
-        llmk_layernorm_backward(dresidual, dl_ln2w, dl_ln2b, scratchF, dl_btc, l_residual2, l_ln2w, l_ln2_mean, l_ln2_rstd, (int)B, (int)T, (int)C, st);
+        layernorm_backward((int)L + l, dl_ln2w, dl_ln2b, dl_btc, l_residual2, l_ln2w, l_ln2_mean, l_ln2_rstd);
         llmk_matmul_backward(dl_btc, dl_attprojw, dl_attprojb, dresidual, l_atty, l_attprojw, scratchF, (int)B, (int)T, (int)C, (int)C, st, nullptr, 1);
         llmk_attention_backward(dl_bt4c, dl_btc, l_qkvr, l_atty, l_att, (int)B, (int)T, (int)NH, (int)C, st);
         if (R >= 2) llmk_layernorm_forward(l_ln1, l_ln1_mean, l_ln1_rstd, residual, l_ln1w, l_ln1b, (int)B, (int)T, (int)C, st);
         llmk_matmul_backward(dl_btc, dl_qkvw, dl_qkvb, dl_bt4c, l_ln1, l_qkvw, scratchF, (int)B, (int)T, (int)C, (int)(3 * C), st, nullptr, 1);
-        llmk_layernorm_backward(dresidual, dl_ln1w, dl_ln1b, scratchF, dl_btc, residual, l_ln1w, l_ln1_mean, l_ln1_rstd, (int)B, (int)T, (int)C, st);
+        layernorm_backward(l, dl_ln1w, dl_ln1b, dl_btc, residual, l_ln1w, l_ln1_mean, l_ln1_rstd);
         // gradient exchange with other GPUs would be launched here (train_gpt2.cu:929-947); one GPU: nothing to do
     }
+    if (ln_together) llmk::layernorm_backward_reduce(ln_grads, num_ln, ln_partials, ln_blocks, (int)C, st);
     llmk_encoder_backward(g.wte, g.wpe, a.output, m->workload_indices, m->bucket_info, dresidual, m->inputs, inputs,
                           (int)B, (int)T, (int)C, llmk::random_u32(&m->rng_state), st);
     if (last_step) llmk_global_sum_deterministic(m->accumulated_mean_loss, a.losses, (int)(B * T), st);

@@ -143,6 +143,45 @@ def test_fp32_small_model_vs_oracle_all_modes(recompute, gelu_fusion):
     m.free()
 
 
+@pytest.mark.parametrize("layers,channels,B,T,Vp", [
+    (1, 64, 1, 1, 320),            # one row, one layer
+    (12, 128, 4, 50, 128),         # more partial sums than the logits buffer holds: each LayerNorm added up on its own
+    (5, 192, 3, 37, 2048),         # ten workgroups of rows, all LayerNorms in one launch
+])
+@pytest.mark.parametrize("precision", ["bf16", "fp32"])
+def test_layernorm_gradients_of_every_layer(precision, layers, channels, B, T, Vp):
+    """Every LayerNorm's dweight and dbias land at that LayerNorm, whether their partial sums are added up together or one by
+    one, and add to what an earlier micro-step left. Against the oracle, each LayerNorm by itself: fp32 1e-3 of its largest
+    element as for every tensor of the fp32 tests. bf16: two accumulated micro-steps on the same batch are twice the one
+    step at half the loss, exactly but for the roundings of one sum (2^-8) and of two (2^-9 + 2^-8): 2.5 * 2^-8."""
+    cfg = ol.Config(64, Vp - 20, Vp, layers, channels // 64, channels)
+    params = ol.init_params(cfg, 5)
+    params += (np.random.RandomState(1).standard_normal(params.size) * 0.02).astype(np.float32)
+    sizes, _ = ol.param_sizes(cfg)
+    params[:sizes[0]].reshape(Vp, channels)[cfg.vocab_size:] = 0
+    inp, tgt = ol.make_tokens(B, T, cfg.vocab_size, 3)
+    m = Model(precision, cfg, B, T, params=params)
+    L, p = m.L, lambda a: a.ctypes.data_as(C.c_void_p)
+
+    def grads(micro_steps):
+        for k in range(micro_steps):
+            L.gpt2_forward(m.h, p(inp), B, T)
+            L.gpt2_backward_and_reduce(m.h, p(inp), p(tgt), micro_steps, k)
+        g, offs = m.grads(), np.cumsum([0] + sizes)
+        return {NAMES[i]: g[offs[i]:offs[i + 1]].reshape(-1, channels) for i in (2, 3, 8, 9, 14, 15)}
+    one, two = grads(1), grads(2)
+    m.free()
+    if precision == "fp32":
+        ref, offs = ol.cref_train(cfg, params, inp, tgt, B, T, 1, lr=0.0, grad_step=0)["grads"], np.cumsum([0] + sizes)
+        want, bound = {NAMES[i]: ref[offs[i]:offs[i + 1]].reshape(-1, channels) for i in (2, 3, 8, 9, 14, 15)}, 1e-3
+    else:
+        want, bound = two, 2.5 * 2.0 ** -8
+    for name in one:
+        for got in (one, two):
+            off = np.abs(got[name] - want[name]).max(1) / np.abs(want[name]).max(1)
+            assert off.max() <= bound, (name, off)
+
+
 @pytest.mark.parametrize("heads,channels", [(16, 1024), (25, 1600), (16, 1536), (4, 512)])
 def test_wider_gpt2_layers_vs_oracle(heads, channels):
     # the layer widths of GPT-2 350M (d24) and 1558M (d48), and of GPT-3's 760M descriptor (head size 96,
@@ -491,8 +530,8 @@ def test_bf16_generation_samples_from_its_own_logits():
     ("fp32", (160, 300, 320, 2, 2, 128), 150, 70),
 ])
 def test_generation_by_blocks_is_the_full_forward_pass(precision, cfg, T, genT):
-    """Every draw of gpt2_generate runs the block of 32 rows that its position lies in, on the K and V kept from the rows
-    before. Each token has to be the sampler's answer for that position's logits of a full forward pass over the finished
+    """Every draw of gpt2_generate runs the one row of its position on the K and V kept from the rows before (attention
+    takes the 32 rows the position lies in). Each token has to be the sampler's answer for that position's logits of a full forward pass over the finished
     sequence. Against the full pass the bf16 logits may round differently (other kernels, other order of sums), which
     moves a token only when a coin falls within that rounding of a boundary of the distribution: 3 of them at most, and none
     in fp32."""
