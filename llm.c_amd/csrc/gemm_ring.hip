@@ -394,7 +394,11 @@ double launch_us(const TileCost& c, int layout, int M, int N, int K, int splits,
 // writing and adding up the fp32 partial products
 double reduce_us(int M, int N, int splits) { return 3.5 + (double)M * N * 8.0 * splits / 5e6; }
 constexpr int MIN_STAGES = 4;            // fewest stages of a piece of K
-constexpr double STAY = 0.96;            // what a ring launch has to come down to before it replaces the persistent kernel
+// What a ring launch's estimate has to come down to before it replaces the persistent kernel. Where the weight gradients of the two
+// are estimated within a tenth the persistent kernel was as good or better (dinp and dweight, us, persistent / ring: 1024 x 1024 over
+// 16384 rows, estimated at 0.91, 94.1 / 95.0; 768 x 768 over 32768, 0.96, 120.4 / 121.9; on the other side 1280 x 1280 over 8192,
+// 0.90, 107 / 87; 768 x 768 over 24576, 0.87, 102.7 / 99.7 and over 16384, 0.82, 83.6 / 69.5).
+constexpr double STAY = 0.96, STAY_DWEIGHT = 0.905;
 }  // namespace
 
 GemmPlan plan_gemm(int layout, int M, int N, int K, int max_splits, bool small_tiles, double persistent_us, int num_cu) {
@@ -413,7 +417,7 @@ GemmPlan plan_gemm(int layout, int M, int N, int K, int max_splits, bool small_t
         }
     }
     const int stages = CEIL_DIV(K, RING_K);
-    double least = best.us * STAY;
+    double least = best.us * (layout == 2 ? STAY_DWEIGHT : STAY);
     for (int c = 0; c < RING_CFGS; c++) {
         const size_t tiles = (size_t)CEIL_DIV(M, RING_COST[c].bm) * CEIL_DIV(N, RING_COST[c].bn);
         if (tiles > (size_t)num_cu * 4096) continue;                // (a grid of 32 bits)
