@@ -29,8 +29,8 @@
  *     message and return instead, for tests; read it with llmk_last_error().
  *
  * Shape preconditions: C % 8 == 0 (bf16) / C % 4 == 0 (fp32) for every row length,
- * head size up to 128 for attention (the bf16 build's MFMA kernels cover 64, the size of every
- * GPT-2 model; other sizes take one-wave-per-row kernels), 16-byte aligned pointers.
+ * head size up to 128 for attention (the MFMA kernels cover 64, the size of every GPT-2 model, 80, 96 and 128 in the bf16
+ * build and 32, 64, 96 and 128 in the fp32 one; other sizes take one-wave-per-row kernels), 16-byte aligned pointers.
  */
 #ifndef LLMK_H
 #define LLMK_H

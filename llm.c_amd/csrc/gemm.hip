@@ -272,7 +272,7 @@ void launch_gemm(const GemmArgs& g, int splits, bool big, hipStream_t st) {
 constexpr int K_ALIGN = 8;       // K-contiguous rows are read in 16-byte chunks
 constexpr int BIG_TILE = 256, SMALL_TILE = 128, K_STEP = 64;
 
-// Persistent direct-to-LDS kernel (gemm_pipelined.hpp). Preconditions: K and the per-split K multiples of 32,
+// Persistent direct-to-LDS kernel (gemm_pipelined.hpp). Preconditions: K and the per-split K multiples of 64,
 // leading dimensions and N multiples of 8, 16-byte aligned operands, 8-byte aligned bias.
 bool pipelined_ok(const GemmArgs& g) { return g.K % KGRAN == 0 && g.k_per_split % KGRAN == 0 && operands_ok(g); }
 // The pipelined kernel's += epilogue spills registers (it holds the old values of a whole tile); with it available,
